@@ -185,6 +185,12 @@ int check_launch(const char* what);
 int quant_rows_fp8(const void* src, int src_dtype, int64_t rows, int64_t cols, int64_t ld, void* dst, float* scale,
                    const int* row_limit, hipStream_t s);
 
+// ---- the forward products for few rows per expert (csrc/gemm_small.hip); elem: bytes of a value (2 bf16, 4 fp32) ----
+bool swiglu_small_takes(int64_t R, int64_t H, int64_t F, int64_t E, int elem);
+int swiglu_small_fwd(bool f32, const void* xp, const void* w_gate, const void* w_up, const void* w_down,
+                     const int* offsets, int64_t R, int64_t H, int64_t F, int64_t E, void* act, void* hgu, void* y,
+                     hipStream_t s);
+
 // ---- optional per-kernel timing (host side; off unless moe_prof_enable(1)) ----
 // Brackets one launch with two hipEvents recorded on the launch stream.
 struct ProfScope {

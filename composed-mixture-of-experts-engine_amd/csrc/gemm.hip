@@ -1102,6 +1102,8 @@ extern "C" int moe_swiglu_fwd(const void* xp, const void* w_gate, const void* w_
     return fail_arg("moe_swiglu_fwd: null or misaligned pointer");
   if (ws_bytes < moe_swiglu_workspace(E) || !workspace) return set_error("moe_swiglu_fwd: workspace"), MOE_EWORKSPACE;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (swiglu_small_takes(R, H, F, E, 2))
+    return swiglu_small_fwd(false, xp, w_gate, w_up, w_down, offsets, R, H, F, E, act, hgu, y, s);
   int* tile_off = static_cast<int*>(workspace);
   int* korder = tile_off + (E + 1);
   MOE_LAUNCH("k_gemm_tiles", k_gemm_tiles, dim3(1), dim3(1024), 0, s, offsets, (int)E, kTileBM, tile_off, korder);

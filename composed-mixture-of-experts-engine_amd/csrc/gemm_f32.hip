@@ -323,6 +323,8 @@ extern "C" int moe_swiglu_fwd_f32(const float* xp, const float* w_gate, const fl
   if (!workspace || ws_bytes < moe_swiglu_f32_workspace(E))
     return set_error("moe_swiglu_fwd_f32: workspace"), MOE_EWORKSPACE;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (a16f(act) && a16f(y) && (!hgu || a16f(hgu)) && swiglu_small_takes(R, H, F, E, 4))
+    return swiglu_small_fwd(true, xp, w_gate, w_up, w_down, offsets, R, H, F, E, act, hgu, y, s);
   int* tile_off = static_cast<int*>(workspace);
   MOE_LAUNCH("k_gemm_tiles_f32", k_gemm_tiles_f32, dim3(1), dim3(64), 0, s, offsets, (int)E, tile_off);
   GemmF32Args a{};
