@@ -88,6 +88,8 @@ struct GemmArgs {
   uint8_t* aqs;        // ... and its E8M0 block scales, slice-major: [(f / 128) * srows + row] * 4 + (f / 32) % 4
   const uint8_t* mxs;  // mode 2, EPI0: the A operand's E8M0 block scales in that layout (A's rows are act's)
   int64_t srows;       // rows per slice of the block-scale layout (a multiple of 4)
+  float* part;         // row-grouped EPI0: partial tiles of the split last round (null: no split)
+  int npart;           // ... and how many of them an XCD has room for
   int E;
   int M, N, K;         // k-grouped: M, N fixed; row-grouped: N, K fixed
 };
@@ -213,7 +215,35 @@ __device__ __forceinline__ int mx_exponent(float amax) {
   return e < -127 ? -127 : (e > 127 ? 127 : e);
 }
 
-template <int AMODE, int BMODE, int GROUP, int EPI, int NW>
+// The last round of a row-grouped product.  An XCD's range of n tiles runs on its 32 CUs, one block each, so its last
+// n % 32 tiles leave the rest of the XCD idle for a whole tile's time; with few rows (a prompt of 1000 tokens through
+// E = 8, H = 4096 has 128 tiles in all, 16 an XCD) that round is the whole product.  Those tiles are split over their
+// k slices instead: each of the r = n % 32 becomes S blocks of about nk / S slices, whose fp32 tiles go to
+// memory and are summed in split order by k_gemm_reduce.  S (1 to 8, r S at most npart) is the one with
+// the least estimated time in slices (about 1.35 us each): the rounds that r S blocks take, plus writing and reading
+// back a partial tile (256 KB each way at a CU's share of the memory rate: 20 slices), plus the reduction's launch.
+// Every block computes it from the device's tile count; the reduction does the same.
+constexpr int kSplitMax = 64;
+__device__ __forceinline__ int split_of(int n, int nk, int npart) {
+  const int r = n & 31;
+  int best = 1, cost = nk;
+  for (int S = 2; S <= 8; ++S) {
+    if (r * S > npart || S > nk) break;
+    const int c = ((r * S + 31) >> 5) * ((nk + S - 1) / S + 20) + 5;
+    if (c < cost) {
+      cost = c;
+      best = S;
+    }
+  }
+  return r ? best : 1;
+}
+
+// Which blocks of a split product a launch runs.  The 8-wave form runs both kinds in one launch; in the 4-wave form,
+// whose main loop takes every register there is, the parts' code costs the loop spills (fp8 347 -> 450 us, bf16 3-6%),
+// so whole tiles and parts are two launches of two instantiations.
+enum { kWhole = 1, kParts = 2, kBoth = 3 };
+
+template <int AMODE, int BMODE, int GROUP, int EPI, int NW, int RUN>
 __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
   constexpr int GNT = NW * 64;
   constexpr int GWN = NW == 8 ? 64 : 128;
@@ -238,12 +268,34 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
   // tiles any routing can produce; the real tile count is known only on the device, so it is split
   // into 8 equal contiguous ranges (one per XCD: blockIdx mod 8), and the surplus blocks of every XCD
   // exit at once. ----
-  const int xcd = (int)(blockIdx.x & 7), slot = (int)(blockIdx.x >> 3);
+  constexpr bool SPLIT = (RUN & kParts) != 0;
+  static_assert(RUN == kWhole || (GROUP == 0 && EPI == 0), "only plain row-grouped products are split");
+  const int xcd = (int)(blockIdx.x & 7);
+  int slot = (int)(blockIdx.x >> 3);
   int L, e, mbase, mlen, kbase, klen, nt;
+  int ks = 0, ke = 0;        // this block's k slices [ks, ke) when it is one part of a split tile (ke > 0)
+  float* part_out = nullptr;  // ... and where its fp32 tile goes
   if constexpr (GROUP == 0) {
     const int Tn = (EPI == 1) ? (2 * g.F + GBN - 1) / GBN : (g.N + GBN - 1) / GBN;
     const int total = g.tile_off[g.E] * Tn;
     const int chunk = (total + 7) >> 3;
+    if constexpr (EPI == 0) {
+      if (g.part != nullptr) {
+        const int n = min(chunk, total - xcd * chunk);  // this XCD's tiles
+        const int full = n & ~31, nkt = (g.K + GBK - 1) / GBK;
+        const int S = n > 0 ? split_of(n, nkt, g.npart) : 1;
+        if constexpr (RUN == kParts) slot += S > 1 ? full : chunk;
+        if (slot >= full && S > 1) {
+          if constexpr (!SPLIT) return;
+          const int j = slot - full, t = j / S, p = j - t * S;
+          if (t >= n - full) return;
+          slot = full + t;
+          ks = __builtin_amdgcn_readfirstlane(nkt * p / S);
+          ke = __builtin_amdgcn_readfirstlane(nkt * (p + 1) / S);
+          part_out = g.part + (int64_t)(xcd * g.npart + j) * (GBM * GBN);
+        }
+      }
+    }
     L = xcd * chunk + slot;
     if (slot >= chunk || L >= total) return;
     int lo = 0, hi = g.E - 1;  // largest e with tile_off[e] * Tn <= L
@@ -259,8 +311,8 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
     const int mt = local - nt * cnt;
     mbase = g.offsets[e] + mt * GBM;
     mlen = min(GBM, g.offsets[e + 1] - mbase);
-    kbase = 0;
-    klen = g.K;
+    kbase = SPLIT ? ks * GBK : 0;
+    klen = SPLIT && ke > 0 ? min(g.K, ke * GBK) - kbase : g.K;
   } else {
     const int Tm = (g.M + GBM - 1) / GBM, Tn = (g.N + GBN - 1) / GBN;
     const int total = g.E * Tm * Tn;
@@ -292,6 +344,8 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
   const int n0 = nt * GBN;
   const int nlen = (EPI == 1) ? min(GBN, 2 * (g.F - nt * (GBN / 2))) : min(GBN, g.N - n0);
   const int nk = (klen + GBK - 1) / GBK;
+  const bool has_split = GROUP == 0 && BMODE == 1 && g.b_split > 0;  // dxp: the second weight follows at k = bsplit
+  const int bsplit = g.b_split - (GROUP == 0 ? kbase : 0);           // in this block's k (not positive: all second)
 
   // ---- per-lane DMA sources.  Wave instruction j (= QPW*wv + q, q < QPW) of an operand fills bytes
   // [1024 j, 1024 j + 1024) of its stage tile: rows mode -> rows 8j + l/8, slot l%8 (one whole
@@ -328,15 +382,15 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
         const int f = nt * (GBN / 2) + (ic >> 6) * 32 + (ic & 31);
         b_src[q] = (((ic >> 5) & 1) ? g.B2 : g.B) + (int64_t)e * g.b_estride + (int64_t)f * g.ldb + b_kl_[q];
       } else {
-        b_src[q] = g.B + (int64_t)e * g.b_estride + (int64_t)(n0 + ic) * g.ldb + b_kl_[q];
+        b_src[q] = g.B + (int64_t)e * g.b_estride + (int64_t)(n0 + ic) * g.ldb + (SPLIT ? kbase : 0) + b_kl_[q];
       }
     } else {
       b_kl_[q] = 2 * j + (lane >> 5);
       int i = (((lane & 31) ^ ((b_kl_[q] & 3) << 2)) << 3);
       i = i < nlen ? i : 0;
       if constexpr (GROUP == 0) {
-        b_src[q] = g.B + (int64_t)e * g.b_estride + (int64_t)b_kl_[q] * g.ldb + n0 + i;
-        if (g.b_split > 0) b_src2[q] = g.B2 + (int64_t)e * g.b_estride + (int64_t)b_kl_[q] * g.ldb + n0 + i;
+        b_src[q] = g.B + (int64_t)e * g.b_estride + (int64_t)((SPLIT ? kbase : 0) + b_kl_[q]) * g.ldb + n0 + i;
+        if (has_split) b_src2[q] = g.B2 + (int64_t)e * g.b_estride + (int64_t)b_kl_[q] * g.ldb + n0 + i;
       } else {
         b_src[q] = g.B + (int64_t)(kbase + b_kl_[q]) * g.ldb + n0 + i;
       }
@@ -366,7 +420,7 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
     uint8_t* const sb = unit + QPW * wv * 1024;
     const int64_t bld = BMODE != 1 ? 1 : g.ldb;
     bool split = false;
-    if constexpr (BMODE == 1 && GROUP == 0) split = g.b_split > 0 && k0 + GBK > g.b_split;
+    if constexpr (BMODE == 1 && GROUP == 0) split = has_split && k0 + GBK > bsplit;
     if (!split) {
       const int64_t step = (int64_t)k0 * bld;
       if (kfull) {
@@ -378,15 +432,15 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
           lds_dma16(k0 + b_kl(q) < klen ? b_at(q, step) : g_zero16, lds_addr(sb + q * 1024));
       }
     } else {
-      const int64_t step1 = (int64_t)k0 * bld, step2 = (int64_t)(k0 - g.b_split) * bld;
-      if (kfull && k0 >= g.b_split) {
+      const int64_t step1 = (int64_t)k0 * bld, step2 = (int64_t)(k0 - bsplit) * bld;
+      if (kfull && k0 >= bsplit) {
 #pragma unroll
         for (int q = 0; q < QPW; ++q) lds_dma16(b_src2[q] + step2, lds_addr(sb + q * 1024));
       } else {
 #pragma unroll
         for (int q = 0; q < QPW; ++q) {
           const int k = k0 + b_kl(q);
-          const uint16_t* src = k >= klen ? g_zero16 : (k < g.b_split ? b_src[q] + step1 : b_src2[q] + step2);
+          const uint16_t* src = k >= klen ? g_zero16 : (k < bsplit ? b_src[q] + step1 : b_src2[q] + step2);
           lds_dma16(src, lds_addr(sb + q * 1024));
         }
       }
@@ -451,21 +505,21 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
       const int64_t bld = BMODE != 1 ? 1 : g.ldb;
       if (full) {
         if constexpr (BMODE == 1 && GROUP == 0) {
-          if (g.b_split > 0 && k0 >= g.b_split) return b_src2[q] + (int64_t)(k0 - g.b_split) * bld;
+          if (has_split && k0 >= bsplit) return b_src2[q] + (int64_t)(k0 - bsplit) * bld;
         }
         return b_at(q, (int64_t)k0 * bld);
       }
       const int k = k0 + b_kl(q);
       if (k >= klen) return g_zero16;
       if constexpr (BMODE == 1 && GROUP == 0) {
-        if (g.b_split > 0 && k >= g.b_split) return b_src2[q] + (int64_t)(k0 - g.b_split) * bld;
+        if (has_split && k >= bsplit) return b_src2[q] + (int64_t)(k0 - bsplit) * bld;
       }
       return b_at(q, (int64_t)k0 * bld);
     };
     auto slice_full = [&](int kt) {
       const int k0 = kt * GBK;
       bool f = k0 + GBK <= klen;
-      if constexpr (BMODE == 1 && GROUP == 0) f = f && !(g.b_split > 0 && k0 < g.b_split && k0 + GBK > g.b_split);
+      if constexpr (BMODE == 1 && GROUP == 0) f = f && !(has_split && k0 < bsplit && k0 + GBK > bsplit);
       return f;
     };
     typedef __attribute__((address_space(1))) const u32x4 g_u32x4;
@@ -496,12 +550,13 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
       static_assert(MI * NI == 16 && NI == 4 && PA <= 16, "fp8 4-wave slot plan");
       uint8_t* const mx_lds = smem + GSMEM + GSCALE;
       const int mx_r0 = mbase & 3;
+      const uint8_t* const mx_src = MX ? g.mxs + ((int64_t)ks * g.srows + (mbase - mx_r0)) * 4 : nullptr;
       u32x4 st_mx;
       auto gload_x = [&](int kt, int p, bool full) {
         if constexpr (MX) {
           if (p == NP) {  // lanes 32-63 repeat lanes 0-31 (no divergent branch in the slot sequence)
             st_mx = *reinterpret_cast<g_u32x4*>(reinterpret_cast<uintptr_t>(
-                g.mxs + ((int64_t)kt * g.srows + (mbase - mx_r0)) * 4 + (wv * 32 + (lane & 31)) * 16));
+                mx_src + (int64_t)kt * g.srows * 4 + (wv * 32 + (lane & 31)) * 16));
             return;
           }
         }
@@ -732,6 +787,24 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
       __builtin_amdgcn_sched_barrier(0);
     }
     wait_vmcnt<0>();
+  }
+  if constexpr (SPLIT) {
+    if (RUN == kParts || part_out != nullptr) {  // a part of a split tile: fp32, in accumulator order (16 bytes a lane, 1 KB a store)
+      float* po = part_out + wv * (MI * NI * 4) * 256;
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < NI; ++ni) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const f32x16& a = acc[mi][ni];
+            reinterpret_cast<f32x4*>(po + v * 256)[lane] = f32x4{a[4 * v], a[4 * v + 1], a[4 * v + 2], a[4 * v + 3]};
+          }
+          po += 4 * 256;
+          __asm__ volatile("" : "+s"(po));  // one scalar base per block: no vector of addresses held ahead
+        }
+      return;
+    }
   }
   __syncthreads();
 
@@ -1017,6 +1090,47 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
   }
 }
 
+// Sums the parts of the split tiles (k_gemm, split_of) in split order and stores the tile: block (t, y) takes slice
+// y of 8 of the t-th split tile of XCD t / 32 (t % 32 < n % 32), with the column scales of an fp8 product applied as
+// its epilogue does.  Reads what the GEMM has just written (mostly the Infinity Cache).
+template <int NW>
+__global__ __launch_bounds__(256) void k_gemm_reduce(GemmArgs g) {
+  constexpr int NI = NW == 8 ? 2 : 4, MI = 4, NW_N = NW == 8 ? 4 : 2;
+  const int xcd = (int)(blockIdx.x >> 5), t = (int)(blockIdx.x & 31);
+  const int Tn = (g.N + GBN - 1) / GBN;
+  const int total = g.tile_off[g.E] * Tn;
+  const int chunk = (total + 7) >> 3;
+  const int n = min(chunk, total - xcd * chunk);
+  if (n <= 0 || t >= (n & 31)) return;
+  const int S = split_of(n, (g.K + GBK - 1) / GBK, g.npart);
+  if (S == 1) return;
+  const int L = xcd * chunk + (n & ~31) + t;
+  int lo = 0, hi = g.E - 1;  // as k_gemm's tile decode
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (g.tile_off[mid] * Tn <= L) lo = mid;
+    else hi = mid - 1;
+  }
+  const int e = lo, cnt = g.tile_off[e + 1] - g.tile_off[e], local = L - g.tile_off[e] * Tn;
+  const int nt = local / cnt, mt = local - nt * cnt;
+  const int mbase = g.offsets[e] + mt * GBM, mlen = min(GBM, g.offsets[e + 1] - mbase);
+  const f32x4* const src = reinterpret_cast<const f32x4*>(g.part + (int64_t)(xcd * g.npart + t * S) * (GBM * GBN));
+  constexpr int U = GBM * GBN / 4;  // 16-byte units of a tile
+  for (int u = (int)blockIdx.y * (U / 8) + threadIdx.x; u < (int)(blockIdx.y + 1) * (U / 8); u += 256) {
+    // unit: wave, (mi, ni), v, lane, as k_gemm stores them
+    const int lane = u & 63, v = (u >> 6) & 3, blk = (u >> 8) % (MI * NI), wv = (u >> 8) / (MI * NI);
+    const int r0 = (wv / NW_N) * GWM + (blk / NI) * 32 + v * 8 + (lane >> 5) * 4;
+    const int c = nt * GBN + (wv % NW_N) * (NI * 32) + (blk % NI) * 32 + (lane & 31);
+    if (r0 >= mlen || c >= g.N) continue;
+    f32x4 s = src[u];
+    for (int p = 1; p < S; ++p) s += src[(int64_t)p * U + u];
+    const float sc = g.sb != nullptr ? g.sb[(int64_t)e * g.N + c] : 1.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (r0 + j < mlen) g.C[(int64_t)(mbase + r0 + j) * g.ldc + c] = f2bf(s[j] * sc);
+  }
+}
+
 // tile_off[0] = 0, tile_off[e+1] = sum_{e' <= e} ceil(rows_e' / bm)  (one block, E <= 1024), and the
 // expert order of the k-grouped products: experts ranked by rows (descending, lower id first on a tie) are
 // dealt to the 8 XCD ranges in snake order (rank r -> range r % 8 on even rounds, 7 - r % 8 on odd ones),
@@ -1074,8 +1188,37 @@ int launch(const char* name, hipStream_t s, const GemmArgs& a, int64_t R) {
     blocks = (int64_t)a.E * ((a.M + GBM - 1) / GBM) * ((a.N + GBN - 1) / GBN);
   }
   if (blocks <= 0) return 0;
-  MOE_LAUNCH(name, (k_gemm<AM, BMD, GR, EP, NW>), dim3(round8(blocks)), dim3(NW * 64), 0, s, a);
+  const dim3 block(NW * 64);
+  if constexpr (GR == 0 && EP == 0) {
+    if (a.part != nullptr) {
+      if constexpr (NW == 8) {
+        MOE_LAUNCH(name, (k_gemm<AM, BMD, GR, EP, NW, kBoth>), dim3(round8(blocks) + 8 * a.npart), block, 0, s, a);
+      } else {
+        MOE_LAUNCH(name, (k_gemm<AM, BMD, GR, EP, NW, kWhole>), dim3(round8(blocks)), block, 0, s, a);
+        MOE_LAUNCH("k_gemm_parts", (k_gemm<AM, BMD, GR, EP, NW, kParts>), dim3(8 * a.npart), block, 0, s, a);
+      }
+      MOE_LAUNCH("k_gemm_reduce", k_gemm_reduce<NW>, dim3(8 * 32, 8), dim3(256), 0, s, a);
+      return check_launch(name);
+    }
+  }
+  MOE_LAUNCH(name, (k_gemm<AM, BMD, GR, EP, NW, kWhole>), dim3(round8(blocks)), block, 0, s, a);
   return check_launch(name);
+}
+
+// Room for the partial tiles of an XCD, for a product of R rows and N columns: 8 a tile, at most kSplitMax.
+int split_parts(int64_t R, int64_t E, int64_t N) {
+  const int64_t tiles = ((R + GBM - 1) / GBM + E) * ((N + GBN - 1) / GBN);
+  return (int)std::min<int64_t>(kSplitMax, 8 * ((tiles + 7) / 8));
+}
+size_t split_bytes(int64_t R, int64_t E, int64_t N) {
+  return (size_t)8 * split_parts(R, E, N) * GBM * GBN * sizeof(float);
+}
+// The caller's workspace past its first `used` bytes, for the partial tiles; too small: the product is not split.
+// Neither is one of 16 rounds of tiles or more, of which the last is too little to pay for the extra launches.
+void take_split(GemmArgs& a, int64_t R, void* ws, size_t ws_bytes, size_t used) {
+  if (R / GBM * ((a.N + GBN - 1) / GBN) >= 16 * 256 || ws_bytes < used + split_bytes(R, a.E, a.N)) return;
+  a.part = reinterpret_cast<float*>(static_cast<char*>(ws) + used);
+  a.npart = split_parts(R, a.E, a.N);
 }
 
 constexpr int kTileBM = GBM;
@@ -1089,6 +1232,10 @@ constexpr int kNW_fwd1 = 4, kNW_fwd2 = 4, kNW_dact = 8, kNW_dxp = 8, kNW_dwd = 8
 using namespace moe;
 
 extern "C" size_t moe_swiglu_workspace(int64_t E) { return (size_t)((2 * E + 1) * 4 + 255) & ~(size_t)255; }
+
+extern "C" size_t moe_swiglu_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E) {
+  return R > 0 && E > 0 && !swiglu_small_takes(R, H, F, E, 2) ? split_bytes(R, E, H) : 0;
+}
 
 extern "C" int moe_swiglu_fwd(const void* xp, const void* w_gate, const void* w_up, const void* w_down,
                               const int32_t* offsets, int64_t R, int64_t H, int64_t F, int64_t E, void* act,
@@ -1140,6 +1287,7 @@ extern "C" int moe_swiglu_fwd(const void* xp, const void* w_gate, const void* w_
   b.ldc = H;
   b.N = (int)H;
   b.K = (int)F;
+  take_split(b, R, workspace, ws_bytes, moe_swiglu_workspace(E));
   return launch<0, 0, 0, 0, kNW_fwd2>("k_gemm_swiglu_fwd2", s, b, R);
 }
 
@@ -1222,6 +1370,7 @@ extern "C" int moe_swiglu_fwd_fp8(const void* xq, const float* sx, const void* w
   b.ldc = H;
   b.N = (int)H;
   b.K = (int)(F / 2);
+  take_split(b, R, workspace, ws_bytes, moe_swiglu_fwd_fp8_workspace(R, F, E));
   return launch<2, 2, 0, 0, kNW_fp8>("k_gemm_swiglu_fwd2_fp8", s, b, R);
 }
 
@@ -1277,6 +1426,7 @@ extern "C" int moe_swiglu_bwd(const void* dy, const void* xp, const void* act, c
     a.ldc = H;
     a.N = (int)H;
     a.K = (int)(2 * F);
+    take_split(a, R, workspace, ws_bytes, moe_swiglu_workspace(E));
     if (int rc = launch<0, 1, 0, 0, kNW_dxp>("k_gemm_swiglu_dxp", s, a, R)) return rc;
   }
   // dWd_e = dy_e^T . act_e   (M = H, N = F, K = rows of e)

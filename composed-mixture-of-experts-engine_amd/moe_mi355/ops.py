@@ -448,7 +448,8 @@ def swiglu_forward(xp: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w
     hgu = torch.empty((R, 2 * F), dtype=xp.dtype, device=dev) if keep_preact else None
     y = torch.empty((R, H), dtype=xp.dtype, device=dev)
     lib = L.load()
-    nbytes = lib.moe_swiglu_f32_workspace(E) if f32 else lib.moe_swiglu_workspace(E)
+    nbytes = lib.moe_swiglu_f32_workspace(E) if f32 else (
+        lib.moe_swiglu_workspace(E) + lib.moe_swiglu_split_workspace(R, H, F, E))
     ws = L.workspace(nbytes, dev)
     fn = lib.moe_swiglu_fwd_f32 if f32 else lib.moe_swiglu_fwd
     rc = fn(xp.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), w_down.data_ptr(), offsets.data_ptr(), R, H, F, E,
@@ -525,7 +526,7 @@ def swiglu_forward_fp8(xq, sx, wq, wscale, offsets, out_dtype=torch.bfloat16, ke
     hgu = torch.empty((R, 2 * F), dtype=out_dtype, device=dev) if keep_preact else None
     y = torch.empty((R, H), dtype=out_dtype, device=dev)
     lib = L.load()
-    nbytes = lib.moe_swiglu_fwd_fp8_workspace(R, F, E)
+    nbytes = lib.moe_swiglu_fwd_fp8_workspace(R, F, E) + lib.moe_swiglu_split_workspace(R, H, F, E)
     ws = L.workspace(nbytes, dev)
     rc = lib.moe_swiglu_fwd_fp8(
         xq.data_ptr(), sx.contiguous().data_ptr(), wg.data_ptr(), sg.contiguous().data_ptr(), wu.data_ptr(),
@@ -559,7 +560,8 @@ def swiglu_backward(dy, xp, act, hgu, w_gate, w_up, w_down, offsets):
     dwu = torch.empty_like(w_up)
     dwd = torch.empty_like(w_down)
     lib = L.load()
-    nbytes = lib.moe_swiglu_f32_workspace(E) if f32 else lib.moe_swiglu_workspace(E)
+    nbytes = lib.moe_swiglu_f32_workspace(E) if f32 else (
+        lib.moe_swiglu_workspace(E) + lib.moe_swiglu_split_workspace(R, H, F, E))
     ws = L.workspace(nbytes, dev)
     fn = lib.moe_swiglu_bwd_f32 if f32 else lib.moe_swiglu_bwd
     rc = fn(dy.data_ptr(), xp.data_ptr(), act.data_ptr(), hgu.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(),

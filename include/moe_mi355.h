@@ -250,6 +250,10 @@ int moe_unpermute_sum(const void* dxp, const void* addend, int dtype, const int3
  * Limits: H % 8 == 0, F % 32 == 0, E <= 1024.
  * ---------------------------------------------------------------------- */
 size_t moe_swiglu_workspace(int64_t E);
+/* Bytes that moe_swiglu_fwd, moe_swiglu_bwd and moe_swiglu_fwd_fp8 use beyond their own workspace size, if the
+ * caller passes that much more (ws_bytes): partial tiles of products whose last round of tiles is split over k.
+ * Without them the same products run unsplit. */
+size_t moe_swiglu_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E);
 int moe_swiglu_fwd(const void* xp, const void* w_gate, const void* w_up, const void* w_down,
                    const int32_t* offsets, int64_t R, int64_t H, int64_t F, int64_t E,
                    void* act, void* hgu, void* y, void* workspace, size_t ws_bytes, void* stream);

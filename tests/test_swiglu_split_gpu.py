@@ -1,0 +1,99 @@
+"""Row-grouped products whose last round of tiles is split over k (csrc/gemm.hip, split_of): the split product against
+the same call without room for its partial tiles, where the tiles run whole, and both against float64."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from gpu_util import dev, say
+
+from moe_mi355 import _lib as L
+from moe_mi355 import ops
+
+pytestmark = pytest.mark.gpu
+
+# (H, F, rows of each expert): one or several m-tiles an expert, ragged ones, k past and short of whole 64-wide slices,
+# dxp's change of weights inside a slice (F % 64 == 32) and inside a part, a width that is no multiple of the tile,
+# more tiles than a round (32 an XCD) and far fewer
+CASES = [
+    (256, 4096, [250, 250]),
+    (264, 2080, [300, 1, 0, 256]),
+    (512, 96, [700]),
+    (1032, 3104, [257, 513, 40, 0]),
+    (4096, 1056, [600] * 30),
+]
+
+
+def _call(fn, *args):
+    L.check(fn(*args), "call")
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"H{c[0]}-F{c[1]}-E{len(c[2])}")
+def test_split_products(case):
+    H, Fd, counts = case
+    E, R = len(counts), sum(counts)
+    say(f"[swiglu split] H={H} F={Fd} E={E} R={R}")
+    lib = L.load()
+    more = lib.moe_swiglu_split_workspace(R, H, Fd, E)
+    assert more > 0
+    g = torch.Generator(device=dev()).manual_seed(H + Fd + R)
+
+    def randn(*s, std=1.0):
+        return (torch.randn(*s, generator=g, device=dev()) * std).to(torch.bfloat16)
+
+    xp, dy = randn(R, H), randn(R, H)
+    wg, wu, wd = randn(E, Fd, H, std=H**-0.5), randn(E, Fd, H, std=H**-0.5), randn(E, H, Fd, std=Fd**-0.5)
+    offs = torch.tensor([0] + counts).cumsum(0).int().to(dev())
+    act, hgu, y = ops.swiglu_forward(xp, wg, wu, wd, offs)
+    dxp, dwg, dwu, dwd = ops.swiglu_backward(dy, xp, act, hgu, wg, wu, wd, offs)
+    # the same with the least workspace that the calls accept
+    n = lib.moe_swiglu_workspace(E)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev())
+    act0, hgu0, y0, dh, dxp0 = (torch.empty_like(t) for t in (act, hgu, y, hgu, dxp))
+    s = L.stream_of(dev())
+    p = [t.data_ptr() for t in (wg, wu, wd, offs)]
+    _call(lib.moe_swiglu_fwd, xp.data_ptr(), *p, R, H, Fd, E, act0.data_ptr(), hgu0.data_ptr(), y0.data_ptr(),
+          ws.data_ptr(), n, s)
+    dws = [torch.empty_like(t) for t in (wg, wu, wd)]
+    _call(lib.moe_swiglu_bwd, dy.data_ptr(), xp.data_ptr(), act0.data_ptr(), hgu0.data_ptr(), *p, R, H, Fd, E,
+          dh.data_ptr(), dxp0.data_ptr(), *[t.data_ptr() for t in dws], ws.data_ptr(), n, s)
+    torch.cuda.synchronize()
+    assert torch.equal(act, act0) and torch.equal(hgu, hgu0)
+    assert all(torch.equal(a, b) for a, b in zip((dwg, dwu, dwd), dws))
+    # a product of n fp32 terms in any order is within n 2^-24 of the sum of their magnitudes, and rounds once to bf16
+    for e in range(E):
+        lo, hi = int(offs[e]), int(offs[e + 1])
+        if lo == hi:
+            continue
+        a, d = act[lo:hi].double(), wd[e].double()
+        h, w1 = dh[lo:hi].double(), torch.cat([wg[e], wu[e]]).double()
+        for got, other, l, r in ((y, y0, a, d.t()), (dxp, dxp0, h, w1)):
+            want = l @ r
+            bound = 2.0**-8 * want.abs() + l.shape[1] * 2.0**-24 * (l.abs() @ r.abs()) + 1e-30
+            for t in (got, other):
+                assert bool(((t[lo:hi].double() - want).abs() <= bound).all())
+
+
+def test_split_fp8():
+    """The e4m3 down projection, split and whole: the same sums in another order, so within one bf16 rounding."""
+    H, Fd, counts = 1024, 4096, [300, 17, 0, 511]
+    E, R = len(counts), sum(counts)
+    g = torch.Generator(device=dev()).manual_seed(7)
+    ws = [torch.randn(E, Fd, H, generator=g, device=dev()) * H**-0.5, torch.randn(E, Fd, H, generator=g, device=dev())
+          * H**-0.5, torch.randn(E, H, Fd, generator=g, device=dev()) * Fd**-0.5]
+    q = [ops.quant_rows_fp8(t.to(torch.bfloat16)) for t in ws]
+    xq, sx = ops.quant_rows_fp8(torch.randn(R, H, generator=g, device=dev()).to(torch.bfloat16))
+    offs = torch.tensor([0] + counts).cumsum(0).int().to(dev())
+    y = ops.swiglu_forward_fp8(xq, sx, tuple(t for t, _ in q), tuple(s for _, s in q), offs, keep_preact=False)[2]
+    lib = L.load()
+    assert lib.moe_swiglu_split_workspace(R, H, Fd, E) > 0
+    n = lib.moe_swiglu_fwd_fp8_workspace(R, Fd, E)
+    wsp = torch.empty(n, dtype=torch.uint8, device=dev())
+    y0 = torch.empty_like(y)
+    _call(lib.moe_swiglu_fwd_fp8, xq.data_ptr(), sx.data_ptr(), *[t.data_ptr() for pair in q for t in pair],
+          offs.data_ptr(), R, H, Fd, E, None, None, y0.data_ptr(), wsp.data_ptr(), n, L.stream_of(dev()))
+    torch.cuda.synchronize()
+    a, b = y.double(), y0.double()
+    # fp32 sums of 4096 terms differ by at most 2 x 4096 x 2^-24 of the sum of magnitudes, here below 8 rms of y
+    assert bool(((a - b).abs() <= 2.0**-7 * b.abs() + 2 * Fd * 2.0**-24 * 8 * b.square().mean().sqrt() * Fd**0.5).all())
