@@ -10,8 +10,9 @@
 // 64-byte half chunk of row r, and the four lanes of a row make one 64-byte request.  The k slot a value lands in
 // is free as long as both operands agree.  Each wave keeps one whole chunk of weights in flight beyond the one it
 // multiplies.  The tokens' fragments come from L2 (re-read by every block).  The waves' partial sums meet in LDS
-// in wave order (fp32), where the SwiGLU is formed with the large kernels' own roundings.  Rows past 32 take
-// further passes over the block's weights.  No tile table: a block finds its rows from `offsets`.
+// in wave order (fp32), where the SwiGLU is formed with the large kernels' own roundings.  Every 32 rows of an expert
+// are a pass of their own blocks over its weights, so a skewed routing's passes run beside each other.  No tile table:
+// a block finds its rows from `offsets`.
 //
 // Blocks start their chunks at different columns (a hash of the block id, wrapping around the row): rows lie a power
 // of two apart, and blocks that walk them in step ask the same few memory channels.  Measured at E = 8, H = 4096,
@@ -37,6 +38,7 @@ struct SmallArgs {
   uint32_t kbytes;     // bytes of a row of A and B
   int N;               // output columns: F (gate/up) or H
   int Tn;              // column tiles
+  int E;
 };
 
 namespace {
@@ -217,40 +219,65 @@ __device__ __forceinline__ void small_pass(const SmallArgs& g, const uint8_t* ba
 template <bool F32, bool GU, int NF, int NW>
 __global__ __launch_bounds__(NW * 64, 8 / NW) void k_gemm_small(SmallArgs g) {
   __shared__ __attribute__((aligned(16))) float red[NW * 16 * (NF * 16 + 4)];
-  const int e = (int)(blockIdx.x / g.Tn), nt = (int)(blockIdx.x % g.Tn);
-  const int lo = g.offsets[e], hi = g.offsets[e + 1];
+  const int slot = (int)(blockIdx.x / g.Tn), nt = (int)(blockIdx.x % g.Tn);
+  int e = slot, pass = 0;
+  if (slot >= g.E) {  // the (slot - E)-th of the passes past the experts' first ones
+    const int lane = threadIdx.x & 63;
+    int x = slot - g.E;
+    for (int e0 = 0;; e0 += 64) {
+      if (e0 >= g.E) return;
+      const int i = e0 + lane;
+      const int c = i < g.E ? max((g.offsets[i + 1] - g.offsets[i] + 31) / 32 - 1, 0) : 0;
+      int upto = c;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(upto, o);
+        upto += lane >= o ? v : 0;
+      }
+      const unsigned long long past = __ballot(x < upto);
+      if (past) {
+        const int l = __builtin_ctzll(past);
+        e = e0 + l;
+        pass = x - (__shfl(upto, l) - __shfl(c, l)) + 1;
+        break;
+      }
+      x -= __shfl(upto, 63);
+    }
+    e = __builtin_amdgcn_readfirstlane(e);
+    pass = __builtin_amdgcn_readfirstlane(pass);
+  }
+  const int m0 = g.offsets[e] + pass * 32, hi = g.offsets[e + 1];
+  if (m0 >= hi) return;
   const int n0 = nt * NF * (GU ? 8 : 16);
   const uint8_t* const b0 = g.B + (int64_t)e * g.b_ebytes;
   const uint8_t* const b1 = GU ? g.B2 + (int64_t)e * g.b_ebytes : nullptr;
-  for (int m0 = lo; m0 < hi; m0 += 32) {
-    if (m0 > lo) __syncthreads();  // the last pass's sums are read
-    if (hi - m0 > 16) small_pass<F32, GU, NF, NW, 2>(g, b0, b1, m0, min(32, hi - m0), n0, red);
-    else small_pass<F32, GU, NF, NW, 1>(g, b0, b1, m0, hi - m0, n0, red);
-  }
+  if (hi - m0 > 16) small_pass<F32, GU, NF, NW, 2>(g, b0, b1, m0, min(32, hi - m0), n0, red);
+  else small_pass<F32, GU, NF, NW, 1>(g, b0, b1, m0, hi - m0, n0, red);
 }
 
 // 64 weight rows and four waves a block; where that leaves fewer than 512 blocks (two a CU), 32 rows and eight
 // waves: fp32 E = 8, H = 1024, F = 4096 (128 blocks of the down projection) 104 -> 77 us.
 template <bool F32, bool GU>
-int launch_small(const char* name, hipStream_t s, SmallArgs a, int64_t E) {
+int launch_small(const char* name, hipStream_t s, SmallArgs a, int64_t E, int64_t R) {
+  a.E = (int)E;
+  const int64_t slots = E + R / 32;  // every expert's first pass, and as many more as R rows can need
   if (cdiv(a.N, GU ? 32 : 64) * E >= 512) {
     a.Tn = cdiv(a.N, GU ? 32 : 64);
-    MOE_LAUNCH(name, (k_gemm_small<F32, GU, 4, 4>), dim3((unsigned)(a.Tn * E)), dim3(256), 0, s, a);
+    MOE_LAUNCH(name, (k_gemm_small<F32, GU, 4, 4>), dim3((unsigned)(a.Tn * slots)), dim3(256), 0, s, a);
   } else {
     a.Tn = cdiv(a.N, GU ? 16 : 32);
-    MOE_LAUNCH(name, (k_gemm_small<F32, GU, 2, 8>), dim3((unsigned)(a.Tn * E)), dim3(512), 0, s, a);
+    MOE_LAUNCH(name, (k_gemm_small<F32, GU, 2, 8>), dim3((unsigned)(a.Tn * slots)), dim3(512), 0, s, a);
   }
   return check_launch(name);
 }
 }  // namespace
 
-// Up to 24 rows an expert on average (bf16; fp32, whose tiles are further from the stream, up to 64): most experts
-// then take one or two passes, and the passes cost less than the large tiles (figures at the top).  A weight slice
-// is addressed by 32-bit byte offsets.
+// Up to 24 rows an expert on average (fp32: 32): few passes past the first, (1 + R / 32E) of the weights' stream at the
+// most (figures at the top).  A weight slice is addressed by 32-bit byte offsets.
 bool swiglu_small_takes(int64_t R, int64_t H, int64_t F, int64_t E, int elem) {
   const int64_t lim = (int64_t)1 << 32;
-  return R <= (elem == 4 ? 64 : 24) * E && H * F * elem < lim && 32 * std::max(H, F) * elem < lim &&
-         E * std::max((F + 15) / 16, (H + 31) / 32) < ((int64_t)1 << 31);
+  return R <= (elem == 4 ? 32 : 24) * E && H * F * elem < lim && 32 * std::max(H, F) * elem < lim &&
+         (E + R / 32) * std::max((F + 15) / 16, (H + 31) / 32) < ((int64_t)1 << 31);
 }
 
 int swiglu_small_fwd(bool f32, const void* xp, const void* w_gate, const void* w_up, const void* w_down,
@@ -267,8 +294,8 @@ int swiglu_small_fwd(bool f32, const void* xp, const void* w_gate, const void* w
   a.C2 = hgu;
   a.kbytes = (uint32_t)(H * elem);
   a.N = (int)F;
-  const int rc = f32 ? launch_small<true, true>("k_gemm_small_fwd1_f32", s, a, E)
-                     : launch_small<false, true>("k_gemm_small_fwd1", s, a, E);
+  const int rc = f32 ? launch_small<true, true>("k_gemm_small_fwd1_f32", s, a, E, R)
+                     : launch_small<false, true>("k_gemm_small_fwd1", s, a, E, R);
   if (rc) return rc;
   SmallArgs b{};
   b.offsets = offsets;
@@ -278,8 +305,8 @@ int swiglu_small_fwd(bool f32, const void* xp, const void* w_gate, const void* w
   b.C = y;
   b.kbytes = (uint32_t)(F * elem);
   b.N = (int)H;
-  return f32 ? launch_small<true, false>("k_gemm_small_fwd2_f32", s, b, E)
-             : launch_small<false, false>("k_gemm_small_fwd2", s, b, E);
+  return f32 ? launch_small<true, false>("k_gemm_small_fwd2_f32", s, b, E, R)
+             : launch_small<false, false>("k_gemm_small_fwd2", s, b, E, R);
 }
 
 }  // namespace moe

@@ -448,14 +448,20 @@ def swiglu_forward(xp: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w
     hgu = torch.empty((R, 2 * F), dtype=xp.dtype, device=dev) if keep_preact else None
     y = torch.empty((R, H), dtype=xp.dtype, device=dev)
     lib = L.load()
-    nbytes = lib.moe_swiglu_f32_workspace(E) if f32 else (
-        lib.moe_swiglu_workspace(E) + lib.moe_swiglu_split_workspace(R, H, F, E))
+    nbytes = _gemm_workspace(lib, f32, R, H, F, E)
     ws = L.workspace(nbytes, dev)
     fn = lib.moe_swiglu_fwd_f32 if f32 else lib.moe_swiglu_fwd
     rc = fn(xp.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), w_down.data_ptr(), offsets.data_ptr(), R, H, F, E,
             act.data_ptr(), L.ptr(hgu), y.data_ptr(), ws.data_ptr(), nbytes, L.stream_of(dev))
     L.check(rc, "moe_swiglu_fwd_f32" if f32 else "moe_swiglu_fwd")
     return act, hgu, y
+
+
+def _gemm_workspace(lib, f32: bool, R: int, H: int, F: int, E: int) -> int:
+    """Bytes of the grouped GEMM's tile tables and of the partial tiles of products split over k."""
+    if f32:
+        return lib.moe_swiglu_f32_workspace(E) + lib.moe_swiglu_f32_split_workspace(R, H, F, E)
+    return lib.moe_swiglu_workspace(E) + lib.moe_swiglu_split_workspace(R, H, F, E)
 
 
 def _gemm_dtype_is_f32(what, *ts) -> bool:
@@ -560,8 +566,7 @@ def swiglu_backward(dy, xp, act, hgu, w_gate, w_up, w_down, offsets):
     dwu = torch.empty_like(w_up)
     dwd = torch.empty_like(w_down)
     lib = L.load()
-    nbytes = lib.moe_swiglu_f32_workspace(E) if f32 else (
-        lib.moe_swiglu_workspace(E) + lib.moe_swiglu_split_workspace(R, H, F, E))
+    nbytes = _gemm_workspace(lib, f32, R, H, F, E)
     ws = L.workspace(nbytes, dev)
     fn = lib.moe_swiglu_bwd_f32 if f32 else lib.moe_swiglu_bwd
     rc = fn(dy.data_ptr(), xp.data_ptr(), act.data_ptr(), hgu.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(),

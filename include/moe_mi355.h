@@ -267,6 +267,7 @@ int moe_swiglu_bwd(const void* dy, const void* xp, const void* act, const void* 
  * moe_layer.py L:166-198, L:326-337).  Limits: H % 4 == 0, F % 32 == 0, E <= 1024; the operands 16-byte
  * aligned.  Workspace: moe_swiglu_f32_workspace(E) bytes. */
 size_t moe_swiglu_f32_workspace(int64_t E);
+size_t moe_swiglu_f32_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E); /* as moe_swiglu_split_workspace */
 int moe_swiglu_fwd_f32(const float* xp, const float* w_gate, const float* w_up, const float* w_down,
                        const int32_t* offsets, int64_t R, int64_t H, int64_t F, int64_t E,
                        float* act, float* hgu, float* y, void* workspace, size_t ws_bytes, void* stream);

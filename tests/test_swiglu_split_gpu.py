@@ -97,3 +97,58 @@ def test_split_fp8():
     a, b = y.double(), y0.double()
     # fp32 sums of 4096 terms differ by at most 2 x 4096 x 2^-24 of the sum of magnitudes, here below 8 rms of y
     assert bool(((a - b).abs() <= 2.0**-7 * b.abs() + 2 * Fd * 2.0**-24 * 8 * b.square().mean().sqrt() * Fd**0.5).all())
+
+
+# fp32: a few tiles only, a last round after whole ones (64 blocks an XCD), column tiles that 8 XCDs share and not
+F32_CASES = [
+    (1000, 608, [300, 0, 140, 77]),
+    (1024, 4096, [525, 503, 542, 471]),
+    (260, 2080, [130, 1, 400]),
+]
+
+
+@pytest.mark.parametrize("case", F32_CASES, ids=lambda c: f"H{c[0]}-F{c[1]}-E{len(c[2])}")
+def test_split_products_f32(case):
+    H, Fd, counts = case
+    E, R = len(counts), sum(counts)
+    say(f"[swiglu split f32] H={H} F={Fd} E={E} R={R}")
+    lib = L.load()
+    assert lib.moe_swiglu_f32_split_workspace(R, H, Fd, E) > 0 and R > 64 * E
+    g = torch.Generator(device=dev()).manual_seed(H + Fd + R)
+
+    def randn(*s, std=1.0):
+        return torch.randn(*s, generator=g, device=dev()) * std
+
+    xp, dy = randn(R, H), randn(R, H)
+    wg, wu, wd = randn(E, Fd, H, std=H**-0.5), randn(E, Fd, H, std=H**-0.5), randn(E, H, Fd, std=Fd**-0.5)
+    offs = torch.tensor([0] + counts).cumsum(0).int().to(dev())
+    act, hgu, y = ops.swiglu_forward(xp, wg, wu, wd, offs)
+    dxp, dwg, dwu, dwd = ops.swiglu_backward(dy, xp, act, hgu, wg, wu, wd, offs)
+    n = lib.moe_swiglu_f32_workspace(E)  # the least workspace: whole tiles
+    ws = torch.empty(n, dtype=torch.uint8, device=dev())
+    act0, hgu0, y0, dh, dxp0 = (torch.empty_like(t) for t in (act, hgu, y, hgu, dxp))
+    s = L.stream_of(dev())
+    p = [t.data_ptr() for t in (wg, wu, wd, offs)]
+    _call(lib.moe_swiglu_fwd_f32, xp.data_ptr(), *p, R, H, Fd, E, act0.data_ptr(), hgu0.data_ptr(), y0.data_ptr(),
+          ws.data_ptr(), n, s)
+    dws = [torch.empty_like(t) for t in (wg, wu, wd)]
+    _call(lib.moe_swiglu_bwd_f32, dy.data_ptr(), xp.data_ptr(), act0.data_ptr(), hgu0.data_ptr(), *p, R, H, Fd, E,
+          dh.data_ptr(), dxp0.data_ptr(), *[t.data_ptr() for t in dws], ws.data_ptr(), n, s)
+    torch.cuda.synchronize()
+    # n fp32 terms in any order: within n 2^-24 of the sum of magnitudes; between two orders, twice that
+    for e in range(E):
+        lo, hi = int(offs[e]), int(offs[e + 1])
+        if lo == hi:
+            continue
+        x, a, d = xp[lo:hi].double(), act[lo:hi].double(), wd[e].double()
+        w1 = torch.cat([wg[e], wu[e]]).double()
+        for got, other, l, r in ((hgu, hgu0, x, w1.t()), (y, y0, a, d.t()), (dxp, dxp0, dh[lo:hi].double(), w1)):
+            want, mag = l @ r, l.abs() @ r.abs()
+            bound = (l.shape[1] + 1) * 2.0**-24 * mag + 1e-30
+            if got is y:  # each from its own act, which differs in rounding
+                bound = bound + act0[lo:hi].double().sub(a).abs() @ r.abs()
+            elif got is dxp:  # from dh of the whole tiles: the split's own differs by the rounding of dy . Wd
+                bound = bound + (H + 16) * 2.0**-24 * 4 * mag
+            for t in (got, other):
+                assert bool(((t[lo:hi].double() - want).abs() <= bound).all())
+        assert bool(torch.isfinite(dwg[e]).all()) and bool(torch.allclose(dwd[e], dws[2][e], rtol=0, atol=1e-4))
