@@ -29,12 +29,10 @@ namespace moe {
 
 // ---------------------------------------------------------------------------
 // Gate pack: wg [H, E] bf16 -> wp[c][nt][lane] (16 bytes each) with
-// element j of lane l = wg[c*32 + (l/16)*8 + j][nt*16 + l%16], zero padded.
+// element j of lane l = wg[c*32 + (l/16)*8 + j][nt*16 + l%16], zero padded to nc chunks of 32 rows.
 // ---------------------------------------------------------------------------
-__global__ void k_pack_gate(const uint16_t* __restrict__ wg, int H, int E, int NT, i16x8* __restrict__ wp,
-                            unsigned* __restrict__ ticket) {
-  if (ticket != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0u;
-  const int64_t total = (int64_t)((H + 31) / 32) * NT * 64;
+__global__ void k_pack_gate(const uint16_t* __restrict__ wg, int H, int E, int NT, int nc, i16x8* __restrict__ wp) {
+  const int64_t total = (int64_t)nc * NT * 64;
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
     const int lane = (int)(q & 63);
     const int64_t r = q >> 6;
@@ -617,7 +615,7 @@ __global__ __launch_bounds__(kFinThreads) void k_router_finalize(const int* __re
 }
 
 // ---------------------------------------------------------------------------
-// Forward, streaming form (bf16 x bf16, E <= 32, H % 256 == 0).  Block = 8 waves = TG groups of 16 tokens.
+// Forward, streaming form (bf16 x bf16, E <= 32, H % 8 == 0).  Block = 8 waves = TG groups of 16 tokens.
 // The block's 16*TG token rows are streamed through a ring of kFwdSlots LDS slots, one 256-column slice per
 // slot, by LDS-DMA with whole 128-byte lines and the streaming cache policy (sc1 nt: the tokens are read
 // once); the matching 256 rows of the raw gate [H, E] ride along in the same slot, so the gate needs no
@@ -628,6 +626,9 @@ __global__ __launch_bounds__(kFinThreads) void k_router_finalize(const int* __re
 // go to part_*.  The last block to finish (ticket counter: zero on entry, reset to zero by that block) folds
 // all blocks' partials, so the finalize needs no launch of its own.
 // ---------------------------------------------------------------------------
+
+// 16 zero bytes: the source of the DMA lanes past the last hidden column of a partial slice.
+__device__ __attribute__((aligned(16))) const uint16_t g_zero16r[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 
 typedef __attribute__((address_space(3))) void lds_void_r;
 __device__ __forceinline__ uint32_t lds_addr_r(const void* p) { return (uint32_t)(uintptr_t)(lds_void_r*)p; }
@@ -745,10 +746,25 @@ __global__ __launch_bounds__(512) void k_router_fwd_stream(
     const int b = (GI * wv + q) * 1024 + lane * 16;
     gofs[q] = b < gbytes ? b : 0;
   }
-  const int nsl = H >> 8;
+  const int nsl = (H + 255) >> 8;
   auto slot_ptr = [&](int sl) { return ring + (sl % kFwdSlots) * SLOT; };
   auto issue = [&](int sl) {
     uint8_t* const sp = slot_ptr(sl);
+    if ((sl + 1) * 256 > H) {  // the last slice of H % 256 != 0: columns and gate rows past H are zeros
+#pragma unroll
+      for (int q = 0; q < XI; ++q) {
+        const int u = (lane & 31) ^ ((2 * (XI * wv + q) + (lane >> 5)) & 31);
+        lds_dma16_stream(sl * 256 + u * 8 < H ? xsrc[q] + sl * 256 : g_zero16r, lds_addr_r(sp + (XI * wv + q) * 1024));
+      }
+      const int64_t gend = (int64_t)H * E * 2;  // a multiple of 16 (H % 8 == 0)
+#pragma unroll
+      for (int q = 0; q < GI; ++q) {
+        const int64_t b = (int64_t)sl * gbytes + gofs[q];
+        lds_dma16_stream(b < gend ? reinterpret_cast<const uint8_t*>(wg) + b : (const uint8_t*)g_zero16r,
+                         lds_addr_r(sp + XB + (GI * wv + q) * 1024));
+      }
+      return;
+    }
 #pragma unroll
     for (int q = 0; q < XI; ++q) lds_dma16_stream(xsrc[q] + sl * 256, lds_addr_r(sp + (XI * wv + q) * 1024));
     const uint8_t* gsrc = reinterpret_cast<const uint8_t*>(wg) + (int64_t)sl * gbytes;
@@ -836,7 +852,7 @@ __global__ __launch_bounds__(512) void k_router_fwd_stream(
 
 // ---------------------------------------------------------------------------
 // Forward, wide streaming form (bf16 x bf16, 32 < E <= 256 as NT = 4, 8 or 16 tiles of 16 experts,
-// H % 64 == 0).  With many experts the gate is as large per hidden column as a sizeable batch of token
+// H % 8 == 0).  With many experts the gate is as large per hidden column as a sizeable batch of token
 // rows, so the block is sized to amortise it: 128 token rows per block (8 waves, one 16-token group
 // each).  The block streams 64-column slices through a ring of kSlots LDS slots by LDS-DMA with the
 // streaming cache policy: the x tile (128 rows x 128 bytes, 16-byte units XOR-swizzled by (row >> 1) & 7,
@@ -912,12 +928,20 @@ __global__ __launch_bounds__(512) void k_router_fwd_wide(
     xsrc[q] = x + (int64_t)min(t0 + row, N - 1) * H + u * 8;
   }
   const uint8_t* gsrc = reinterpret_cast<const uint8_t*>(wp) + (P::GI * wv) * 1024 + lane * 16;
-  const int nsl = H >> 6;
+  const int nsl = (H + 63) >> 6;
   auto slot_ptr = [&](int sl) { return ring + (sl % P::kSlots) * P::SLOT; };
   auto issue = [&](int sl) {
     uint8_t* const sp = slot_ptr(sl);
+    if ((sl + 1) * 64 <= H) {
 #pragma unroll
-    for (int q = 0; q < P::XI; ++q) lds_dma16_stream(xsrc[q] + sl * 64, lds_addr_r(sp + (P::XI * wv + q) * 1024));
+      for (int q = 0; q < P::XI; ++q) lds_dma16_stream(xsrc[q] + sl * 64, lds_addr_r(sp + (P::XI * wv + q) * 1024));
+    } else {  // the last slice of H % 64 != 0: columns past H are zeros (as the packed gate's rows are)
+#pragma unroll
+      for (int q = 0; q < P::XI; ++q) {
+        const int u = (lane & 7) ^ (((8 * (P::XI * wv + q) + (lane >> 3)) >> 1) & 7);
+        lds_dma16_stream(sl * 64 + u * 8 < H ? xsrc[q] + sl * 64 : g_zero16r, lds_addr_r(sp + (P::XI * wv + q) * 1024));
+      }
+    }
 #pragma unroll
     for (int q = 0; q < P::GI; ++q)
       lds_dma16_stream(gsrc + (int64_t)sl * P::GB + q * 1024, lds_addr_r(sp + P::XB + (P::GI * wv + q) * 1024));
@@ -965,7 +989,76 @@ __global__ __launch_bounds__(512) void k_router_fwd_wide(
 }
 
 // ---------------------------------------------------------------------------
-// Forward, fp32 x and fp32 gate (E <= 64, H % 4 == 0, x 16-byte aligned).  The gate GEMM runs on
+// Forward for few tokens and many experts (bf16 x bf16, 32 < E <= 256, H % 8 == 0, N up to kSplitTokens).  The wide
+// form's 128-token blocks leave most CUs without one there and stream the whole hidden dim in turn; here a block is
+// one group of 16 tokens and its 8 waves take every 8th 32-column chunk of the hidden dim, with x and the packed gate
+// loaded straight into MFMA fragments.  The partial logit tiles are summed in LDS in wave order, and wave 0 routes.
+// Latency bound (a chain of H / 256 chunk loads a wave); the gate is re-read from L2 by every block, which is what
+// ends its use with more tokens.  H = 2048, E = 128, K = 8, 64 tokens: 36-43 us in the wide form, here 12 us.
+// ---------------------------------------------------------------------------
+constexpr int kSplitTokens = 4096;
+
+template <int NT>
+__global__ __launch_bounds__(512) void k_router_fwd_split(
+    const uint16_t* __restrict__ x, const i16x8* __restrict__ wp, const float* __restrict__ bias, int N, int H,
+    int E, int K, int64_t* __restrict__ idx_out, void* __restrict__ w_out, int w_dt, float* __restrict__ logits_out,
+    float* __restrict__ lse_out, int* __restrict__ part_cnt, float* __restrict__ part_p, float* __restrict__ part_z,
+    unsigned* __restrict__ ticket, float aux_coef, float z_coef, int64_t* __restrict__ cnt_out,
+    float* __restrict__ stats, float* __restrict__ aux_out, float* __restrict__ z_out) {
+  __shared__ f32x4 s_acc[7 * NT * 64];
+  __shared__ float s_tile[NT <= 8 ? 16 * (NT * 16 + 4) : 1];
+  __shared__ int s_cnt[NT * 16];
+  __shared__ float s_p[1][NT * 16];
+  __shared__ float s_z[1];
+  __shared__ int s_nf[1];
+  __shared__ int s_last;
+  __shared__ float s_fin[finalize_scratch_floats<512>()];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, n = lane & 15;
+  const int t0 = blockIdx.x * 16;
+  for (int i = threadIdx.x; i < NT * 16; i += 512) s_cnt[i] = 0;
+
+  const uint16_t* const xr = x + (int64_t)min(t0 + n, N - 1) * H + g * 8;
+  const i16x8* const wb = wp + lane;
+  const int nc = (H + 31) / 32;
+  f32x4 acc[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll(NT <= 4 ? 4 : NT == 8 ? 2 : 1)
+  for (int c = wv; c < nc; c += 8) {
+    // units past H: zeros (their gate rows are packed as zeros)
+    const bool in = c * 32 + g * 8 < H;
+    const i16x8 v = *reinterpret_cast<const i16x8*>(xr + (in ? c * 32 : -g * 8));
+    const i16x8 a = in ? v : i16x8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+      acc[nt] = mfma16x16x32(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, wb[(c * NT + nt) * 64]), acc[nt]);
+  }
+  if (wv > 0) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) s_acc[((wv - 1) * NT + nt) * 64 + lane] = acc[nt];
+  }
+  __syncthreads();
+  if (wv == 0) {
+#pragma unroll 1  // one wave's tiles at a time: all at once would not fit the registers
+    for (int w = 0; w < 7; ++w)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[nt] += s_acc[(w * NT + nt) * 64 + lane];
+    if constexpr (NT <= 8)
+      route_quad<NT>(acc, s_tile, t0, lane, bias, N, E, K, idx_out, w_out, w_dt, logits_out, lse_out, s_cnt, s_p[0],
+                     &s_z[0], &s_nf[0]);
+    else
+      route_group<NT>(acc, t0, lane, bias, N, E, K, idx_out, w_out, w_dt, logits_out, lse_out, s_cnt, s_p[0], &s_z[0],
+                      &s_nf[0]);
+  }
+  __syncthreads();
+  fwd_block_tail<1, NT>(s_cnt, s_p, s_z, s_nf, s_last, s_fin, N, E, K, part_cnt, part_p, part_z, ticket, aux_coef,
+                        z_coef, cnt_out, stats, aux_out, z_out);
+}
+
+// ---------------------------------------------------------------------------
+// Forward, fp32 x and fp32 gate (E <= 256, H % 4 == 0, x 16-byte aligned).  The gate GEMM runs on
 // v_mfma_f32_16x16x4_f32 (fp32 products, fp32 sums), whose 16x16 accumulator layout is the one the bf16
 // kernels route from.  Block = 8 waves = TG groups of 16 tokens x HS = 8 / TG waves per group; wave hp of a
 // group sums its logits over the hp-th contiguous 1/HS of the 16-column chunks of the hidden dim.  Per chunk
@@ -983,8 +1076,8 @@ __global__ __launch_bounds__(512) void k_router_fwd_f32(
     unsigned* __restrict__ ticket, float aux_coef, float z_coef, int64_t* __restrict__ cnt_out,
     float* __restrict__ stats, float* __restrict__ aux_out, float* __restrict__ z_out) {
   constexpr int HS = 8 / TG;
-  constexpr int U = 4;  // chunks per load group
-  __shared__ f32x4 s_acc[(HS > 1 ? HS - 1 : 1) * TG * NT * 64];
+  constexpr int U = NT <= 4 ? 4 : (NT == 8 ? 2 : 1);  // chunks per load group
+  __shared__ f32x4 s_acc[HS > 1 ? (HS - 1) * TG * NT * 64 : 1];
   __shared__ int s_cnt[NT * 16];
   __shared__ float s_p[TG][NT * 16];
   __shared__ float s_z[TG];
@@ -1064,7 +1157,7 @@ __global__ __launch_bounds__(512) void k_router_fwd_f32(
   __syncthreads();  // s_cnt zeroed, partial tiles visible
   if constexpr (HS > 1) {
     if (hp == 0) {
-#pragma unroll
+#pragma unroll(NT <= 4 ? HS : 1)
       for (int q2 = 1; q2 < HS; ++q2)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[nt] += s_acc[(((q2 - 1) * TG + tg) * NT + nt) * 64 + lane];
@@ -1584,7 +1677,7 @@ __global__ __launch_bounds__(256) void k_router_dxdw_bf16(const uint16_t* __rest
 }
 
 // ---------------------------------------------------------------------------
-// Backward 2, streaming form (bf16 x bf16, E <= 32, H % 256 == 0): dx = G wg^T and the dwg partial
+// Backward 2, streaming form (bf16 x bf16, E <= 32, H % 8 == 0): dx = G wg^T and the dwg partial
 // x^T G of one (token chunk, 256 hidden columns) block.  Each wave owns 64 hidden columns and a private
 // LDS tile, so after the chunk's G has been staged (token-major and expert-major) the token loop has no
 // workgroup barrier: per 32-token step the wave writes its x tile to LDS, reads the dwg A operand with
@@ -1637,7 +1730,10 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(NTE ==
 
   // x stream: lane loads rows (lane/8) + 8j of the step, 16-byte chunk lane%8 of the wave's 64 columns
   // (rows past the chunk re-read its last row and are zeroed when written to LDS)
-  const uint16_t* xw = x + col0 + (lane & 7) * 8;
+  // (columns past H read the row's last ones: what they give is not stored)
+  const int lcol = min(col0 + (lane & 7) * 8, H - 8);
+  const bool lin = col0 + (lane & 7) * 8 < H;
+  const uint16_t* xw = x + lcol;
   auto load_x = [&](u32x4(&r)[4], int ts0) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1651,7 +1747,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(NTE ==
     for (int j = 0; j < 4; ++j) {
       const int t = ts0 + (lane >> 3) + 8 * j;
       r[j] = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x4*>(src + col0 + (lane & 7) * 8 + (int64_t)min(t, tend - 1) * H));
+          reinterpret_cast<const u32x4*>(src + lcol + (int64_t)min(t, tend - 1) * H));
     }
   };
   // ---- G = dL/dlogits of the chunk, one token per thread, rounded to bf16 as the reference does
@@ -1744,13 +1840,13 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(NTE ==
   if (E == 8) {  // each gate row is one 16-byte piece (lanes past the first 8 experts hold zeros)
 #pragma unroll
     for (int nc = 0; nc < 4; ++nc) {
-      const i16x8 v = *reinterpret_cast<const i16x8*>(wg + (int64_t)(col0 + nc * 16 + n) * 8);
+      const i16x8 v = *reinterpret_cast<const i16x8*>(wg + (int64_t)min(col0 + nc * 16 + n, H - 1) * 8);
       wB[nc] = g == 0 ? v : i16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
   } else {
 #pragma unroll
     for (int nc = 0; nc < 4; ++nc) {
-      const int h = col0 + nc * 16 + n;
+      const int h = min(col0 + nc * 16 + n, H - 1);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int e = g * 8 + j;
@@ -1817,7 +1913,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(NTE ==
       const int t = tbeg + lr0 + lr;
       u32x4 v = *reinterpret_cast<const u32x4*>(&xsw[lr * kSXP + (lane & 7) * 8]);
       if (dx_add != nullptr) v = add_bf16x8(v, ad[j]);
-      if (t < tend) *reinterpret_cast<u32x4*>(dx + (int64_t)t * H + col0 + (lane & 7) * 8) = v;
+      if (t < tend && lin) *reinterpret_cast<u32x4*>(dx + (int64_t)t * H + lcol) = v;
     }
   };
 
@@ -1835,12 +1931,12 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(NTE ==
       for (int i = 0; i < 4; ++i) {
         const int h = col0 + mt * 16 + g * 4 + i;
         const int e = ne * 16 + n;
-        if (e < E) out[(int64_t)h * E + e] = accw[mt][ne][i];
+        if (e < E && h < H) out[(int64_t)h * E + e] = accw[mt][ne][i];
       }
 }
 
 // ---------------------------------------------------------------------------
-// Backward 2, wide form (bf16 x bf16, 32 < E <= 128 as EK = 2 or 4 chunks of 32 experts, H % 256 == 0):
+// Backward 2, wide form (bf16 x bf16, 32 < E <= 128 as EK = 2 or 4 chunks of 32 experts, H % 8 == 0):
 // dx = G wg^T and the dwg partial x^T G of one (token chunk, 256 hidden columns) block, with G = dL/dlogits
 // in bf16 ([N, EKP], from k_router_glogits).  With many experts the fp32 dwg partials ([chunks, H, E]) are
 // as large as x unless the chunks are long, so each block covers ~N * nht / 256 tokens (about one block
@@ -1884,7 +1980,10 @@ __global__ __launch_bounds__(256) void k_router_dxdw_wide(const uint16_t* __rest
 
   // x stream: lane loads rows (lane/8) + 8j of the step, 16-byte chunk lane%8 of the wave's 64 columns
   // (rows past the chunk re-read its last row and are zeroed when written to LDS)
-  const uint16_t* xw = x + col0 + (lane & 7) * 8;
+  // (columns past H read the row's last ones: what they give is not stored)
+  const int lcol = min(col0 + (lane & 7) * 8, H - 8);
+  const bool lin = col0 + (lane & 7) * 8 < H;
+  const uint16_t* xw = x + lcol;
   auto load_x = [&](u32x4(&r)[4], int ts0) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1898,7 +1997,7 @@ __global__ __launch_bounds__(256) void k_router_dxdw_wide(const uint16_t* __rest
     for (int j = 0; j < 4; ++j) {
       const int t = ts0 + (lane >> 3) + 8 * j;
       r[j] = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x4*>(src + col0 + (lane & 7) * 8 + (int64_t)min(t, tend - 1) * H));
+          reinterpret_cast<const u32x4*>(src + lcol + (int64_t)min(t, tend - 1) * H));
     }
   };
   // G stream: unit q = tid + 256 j of the step is row q / GU, 16-byte unit q % GU
@@ -1931,7 +2030,7 @@ __global__ __launch_bounds__(256) void k_router_dxdw_wide(const uint16_t* __rest
   i16x8 wB[4][EK];
 #pragma unroll
   for (int nc = 0; nc < 4; ++nc) {
-    const uint16_t* wr = wg + (int64_t)(col0 + nc * 16 + n) * E;
+    const uint16_t* wr = wg + (int64_t)min(col0 + nc * 16 + n, H - 1) * E;
 #pragma unroll
     for (int ek = 0; ek < EK; ++ek) {
       const int e0 = ek * 32 + g * 8;
@@ -2007,8 +2106,7 @@ __global__ __launch_bounds__(256) void k_router_dxdw_wide(const uint16_t* __rest
       const int t = tbeg + lr0 + lr;
       u32x4 v = *reinterpret_cast<const u32x4*>(&xsw[lr * kSXP + (lane & 7) * 8]);
       if (dx_add != nullptr) v = add_bf16x8(v, ad[j]);
-      if (t < tend)
-        __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dx + (int64_t)t * H + col0 + (lane & 7) * 8));
+      if (t < tend && lin) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dx + (int64_t)t * H + lcol));
     }
   };
 
@@ -2026,7 +2124,7 @@ __global__ __launch_bounds__(256) void k_router_dxdw_wide(const uint16_t* __rest
       for (int i = 0; i < 4; ++i) {
         const int h = col0 + mt * 16 + g * 4 + i;
         const int e = ne * 16 + n;
-        if (e < E) out[(int64_t)h * E + e] = accw[mt][ne][i];
+        if (e < E && h < H) out[(int64_t)h * E + e] = accw[mt][ne][i];
       }
 }
 
@@ -2102,6 +2200,89 @@ __global__ __launch_bounds__(256) void k_router_dxdw_f32(const float* __restrict
       for (int e = 0; e < EL; ++e)
         if (e < E) dst[i * E + e] = acc[i][e];
   }
+}
+
+// Backward, fp32 x and gate, more experts than k_router_dxdw_f32 holds in registers (16 < E <= 256, E % 4 == 0), on
+// v_mfma_f32_16x16x4_f32 with fragments loaded straight from memory (G, the gate and x all come from L2 after their
+// first read; the products are a few microseconds of MFMA).  N = 2749, H = 1024, E = 64: the step's generic kernels
+// took 790 us, these 20.
+//
+// dx = G wg^T: a wave owns 16 tokens x 64 columns; both operands are contiguous in e, so a lane's 16-byte load holds
+// its row's four k of four MFMAs (k slot q of MFMA s is expert 16 c + 4 q + s for A and B alike).
+__global__ __launch_bounds__(256) void k_router_dx_f32(const float* __restrict__ G, const float* __restrict__ wg, int N,
+                                                       int H, int E, float* __restrict__ dx) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int n = lane & 15, q = lane >> 4;
+  const int t0 = blockIdx.x * 64 + wv * 16, h0 = blockIdx.y * 64;
+  if (t0 >= N) return;
+  const float* const gr = G + (int64_t)min(t0 + n, N - 1) * E + 4 * q;
+  const float* wr[4];
+#pragma unroll
+  for (int f = 0; f < 4; ++f) wr[f] = wg + (int64_t)min(h0 + f * 16 + n, H - 1) * E + 4 * q;
+  f32x4 acc[4];
+#pragma unroll
+  for (int f = 0; f < 4; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int e = 0; e < E; e += 16) {
+    const bool in = e + 4 * q < E;  // units past E: zeros on both sides
+    const int o = in ? e : -4 * q;
+    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    const f32x4 av = *reinterpret_cast<const f32x4*>(gr + o);
+    const f32x4 a = in ? av : z;
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const f32x4 bv = *reinterpret_cast<const f32x4*>(wr[f] + o);
+      const f32x4 b = in ? bv : z;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc[f], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int t = t0 + 4 * q + j, h = h0 + f * 16 + n;
+      if (t < N && h < H) dx[(int64_t)t * H + h] = acc[f][j];
+    }
+}
+
+// dwg partial x^T G of one token chunk: a wave owns 16 columns x all E experts (NTE tiles of 16); per four tokens a
+// lane loads one x value and NTE values of G (64-byte row segments).
+template <int NTE>
+__global__ __launch_bounds__(256) void k_router_dw_f32(const float* __restrict__ x, const float* __restrict__ G, int N,
+                                                       int H, int E, int tc_len, float* __restrict__ ws_dw) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int n = lane & 15, q = lane >> 4;
+  const int h0 = blockIdx.x * 64 + wv * 16;
+  if (h0 >= H) return;
+  const int tbeg = blockIdx.y * tc_len, tend = min(N, tbeg + tc_len);
+  const float* const xc = x + min(h0 + n, H - 1);
+  int ec[NTE];
+#pragma unroll
+  for (int nt = 0; nt < NTE; ++nt) ec[nt] = min(nt * 16 + n, E - 1);
+  f32x4 acc[NTE];
+#pragma unroll
+  for (int nt = 0; nt < NTE; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll(NTE <= 4 ? 4 : 2)
+  for (int t4 = tbeg; t4 < tend; t4 += 4) {
+    const bool in = t4 + q < tend;  // tokens past the chunk: zeros on both sides
+    const int t = min(t4 + q, tend - 1);
+    const float av = xc[(int64_t)t * H];
+    const float a = in ? av : 0.f;
+#pragma unroll
+    for (int nt = 0; nt < NTE; ++nt) {
+      const float bv = G[(int64_t)t * E + ec[nt]];
+      acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, in ? bv : 0.f, acc[nt], 0, 0, 0);
+    }
+  }
+  float* const out = ws_dw + (int64_t)blockIdx.y * H * E;
+#pragma unroll
+  for (int nt = 0; nt < NTE; ++nt)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int h = h0 + 4 * q + j, e = nt * 16 + n;
+      if (h < H && e < E) out[(int64_t)h * E + e] = acc[nt][j];
+    }
 }
 
 // Generic dx = G wg^T: one thread per (t, h).
@@ -2200,10 +2381,11 @@ constexpr int fwd_u(int NT) { return NT <= 4 ? 4 : 2; }
 int fwd_tokens_per_block(int NT) { return 16 * (4 / fwd_hs(NT)); }
 
 struct FwdPlan {
-  bool f32;     // k_router_fwd_f32 (fp32 x and gate, E <= 64, H % 4 == 0)
-  bool mfma;
-  bool stream;  // k_router_fwd_stream (E <= 32, H % 256 == 0)
-  bool wide;    // k_router_fwd_wide (32 < E <= 256, H % 64 == 0)
+  bool f32;     // k_router_fwd_f32 (fp32 x and gate, H % 4 == 0)
+  bool mfma;    // k_router_fwd_bf16 (an unaligned gate; E <= 128, H % 32 == 0)
+  bool stream;  // k_router_fwd_stream (E <= 32, H % 8 == 0)
+  bool wide;    // k_router_fwd_wide, or with few tokens k_router_fwd_split (32 < E <= 256, H % 8 == 0)
+  bool split;
   int NT, TG;
   int nblk;
   size_t off_wp, off_cnt, off_p, off_z, off_ticket, total;
@@ -2211,24 +2393,29 @@ struct FwdPlan {
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// Packed gate: 32-row chunks, a whole number of the wide form's 64-column slices.
+int gate_chunks(int64_t H) { return 2 * (int)((H + 63) / 64); }
+
 FwdPlan plan_fwd(int64_t N, int64_t H, int64_t E, int x_dt, int w_dt, bool allow_stream = true) {
   FwdPlan p{};
   p.mfma = x_dt == MOE_BF16 && w_dt == MOE_BF16 && H % 32 == 0 && E <= 128;
   p.NT = (int)((E + 15) / 16);
   if (p.NT == 3) p.NT = 4;
   if (p.NT > 4 && p.NT < 8) p.NT = 8;
-  p.stream = allow_stream && p.mfma && E <= 32 && H % 256 == 0;
-  p.wide = allow_stream && x_dt == MOE_BF16 && w_dt == MOE_BF16 && E > 32 && E <= kMaxE && H % 64 == 0;
-  p.f32 = allow_stream && x_dt == MOE_F32 && w_dt == MOE_F32 && E <= 64 && H % 4 == 0;
+  const bool rows16 = allow_stream && x_dt == MOE_BF16 && w_dt == MOE_BF16 && H % 8 == 0;
+  p.stream = rows16 && E <= 32;
+  p.wide = rows16 && E > 32 && E <= kMaxE;
+  p.split = p.wide && N <= kSplitTokens;
+  p.f32 = allow_stream && x_dt == MOE_F32 && w_dt == MOE_F32 && E <= kMaxE && H % 4 == 0;
   if (p.f32) {
+    if (p.NT > 8) p.NT = 16;
     // 16 * TG tokens per block: the largest TG that still gives about one block per CU (256)
     const int64_t groups = cdiv(N, 16);
     p.TG = groups >= 256 * 8 ? 8 : (groups >= 256 * 4 ? 4 : (groups >= 256 * 2 ? 2 : 1));
     p.nblk = cdiv(N, 16 * p.TG);
   } else if (p.wide) {
-    p.mfma = true;
     p.NT = E <= 64 ? 4 : (E <= 128 ? 8 : 16);
-    p.nblk = cdiv(N, WideFwd<4>::ROWS);
+    p.nblk = p.split ? cdiv(N, 16) : cdiv(N, WideFwd<4>::ROWS);
   } else if (p.stream) {
     // 16 * TG tokens per block: the largest TG that still gives one block per CU (256)
     p.TG = N >= 256 * 64 ? 4 : (N >= 256 * 32 ? 2 : 1);
@@ -2244,7 +2431,7 @@ FwdPlan plan_fwd(int64_t N, int64_t H, int64_t E, int x_dt, int w_dt, bool allow
   p.off_ticket = off;
   off += 256;
   p.off_wp = off;
-  off += p.mfma ? align256((size_t)((H + 31) / 32) * p.NT * 64 * 16) : 0;
+  off += p.mfma || p.wide ? align256((size_t)gate_chunks(H) * p.NT * 64 * 16) : 0;
   p.off_cnt = off;
   off += align256((size_t)p.nblk * E * sizeof(int));
   p.off_p = off;
@@ -2257,9 +2444,10 @@ FwdPlan plan_fwd(int64_t N, int64_t H, int64_t E, int x_dt, int w_dt, bool allow
 
 struct BwdPlan {
   bool f32;     // k_router_glogits + k_router_dxdw_f32 (fp32 x and gate, E <= 16, H % 4 == 0)
-  bool mfma;
-  bool stream;  // k_router_dxdw_stream (E <= 32, H % 256 == 0)
-  bool wide;    // k_router_glogits + k_router_dxdw_wide (32 < E <= 128, H % 256 == 0)
+  bool f32m;    // k_router_glogits + k_router_dx_f32 + k_router_dw_f32 (fp32 x and gate, E > 16, E % 4 == 0)
+  bool mfma;    // k_router_glogits + k_router_dxdw_bf16 (an unaligned gate; 32 < E <= 128, H % 64 == 0)
+  bool stream;  // k_router_dxdw_stream (E <= 32, H % 8 == 0)
+  bool wide;    // k_router_glogits + k_router_dxdw_wide (32 < E <= 128, H % 8 == 0)
   int EK, NTE;
   int nchunk, tc_len;
   size_t off_g, off_gb, off_ws, total;
@@ -2267,15 +2455,17 @@ struct BwdPlan {
 
 BwdPlan plan_bwd(int64_t N, int64_t H, int64_t E, int x_dt, int w_dt) {
   BwdPlan p{};
-  p.mfma = x_dt == MOE_BF16 && w_dt == MOE_BF16 && H % 64 == 0 && E <= 128;
+  const bool rows16 = x_dt == MOE_BF16 && w_dt == MOE_BF16 && H % 8 == 0;
+  p.mfma = rows16 && H % 64 == 0 && E > 32 && E <= 128;
   p.EK = (int)((E + 31) / 32);
   if (p.EK == 3) p.EK = 4;
   p.NTE = (int)((E + 15) / 16);
   if (p.NTE == 3) p.NTE = 4;
   if (p.NTE > 4 && p.NTE < 8) p.NTE = 8;
-  p.stream = p.mfma && E <= 32 && H % 256 == 0;
-  p.wide = p.mfma && E > 32 && H % 256 == 0;
+  p.stream = rows16 && E <= 32;
+  p.wide = rows16 && E > 32 && E <= 128;
   p.f32 = x_dt == MOE_F32 && w_dt == MOE_F32 && E <= 16 && H % 4 == 0;
+  p.f32m = x_dt == MOE_F32 && w_dt == MOE_F32 && E > 16 && E % 4 == 0;
   if (p.f32) {
     // about 1024 blocks of (256-column slice, token chunk), at most 8 tokens per wave before the chunks grow
     const int64_t nht = cdiv(H, 256);
@@ -2285,7 +2475,7 @@ BwdPlan plan_bwd(int64_t N, int64_t H, int64_t E, int x_dt, int w_dt) {
     p.nchunk = (int)cdiv(N, p.tc_len);
   } else if (p.wide) {
     // about one block per CU; long chunks keep the fp32 dwg partials few
-    const int nht = (int)(H / 256);
+    const int nht = cdiv(H, 256);
     const int want = std::max(1, kWideBwdBlocks / nht);
     p.tc_len = std::max(64, cdiv(cdiv(N, want), 64) * 64);
     p.nchunk = cdiv(N, p.tc_len);
@@ -2293,16 +2483,14 @@ BwdPlan plan_bwd(int64_t N, int64_t H, int64_t E, int x_dt, int w_dt) {
     // one round of blocks: per CU four 4-wave blocks (or one 16-wave block with E <= 8 and H % 1024 == 0)
     // with up to 16 experts (at most 128 registers), two 4-wave blocks with more (the second expert tile's
     // registers); chunks of a multiple of 64 tokens, at most kSTC
-    const int nht = (int)(H / 256);
+    const int nht = cdiv(H, 256);
     const int want = std::max(1, (E <= 16 ? 1024 : 512) / nht);
     p.tc_len = std::min(kSTC, std::max(64, cdiv(cdiv(N, want), 64) * 64));
     p.nchunk = cdiv(N, p.tc_len);
-  } else if (p.mfma) {
-    const int nhb = cdiv(H, 256);
-    int nchunk = std::max(1, 1024 / nhb);
-    const int max_chunks = cdiv(N, kBwdTS);
-    nchunk = std::min(nchunk, max_chunks);
-    p.tc_len = cdiv(cdiv(N, nchunk), kBwdTS) * kBwdTS;
+  } else if (p.f32m) {
+    // about 1024 blocks of (64 columns, token chunk), chunks of at least 64 tokens
+    const int64_t want = std::max<int64_t>(1, 1024 / cdiv(H, 64));
+    p.tc_len = std::max(64, cdiv(cdiv(N, want), 4) * 4);
     p.nchunk = cdiv(N, p.tc_len);
   } else {
     p.tc_len = 256;
@@ -2313,7 +2501,7 @@ BwdPlan plan_bwd(int64_t N, int64_t H, int64_t E, int x_dt, int w_dt) {
   p.off_g = off;  // G (and its bf16 copy) for the non-streaming paths, which an unaligned call falls back to
   off += align256((size_t)N * E * sizeof(float));
   p.off_gb = off;
-  off += p.mfma ? align256((size_t)N * p.EK * 32 * sizeof(uint16_t)) : 0;
+  off += p.wide ? align256((size_t)N * p.EK * 32 * sizeof(uint16_t)) : 0;
   p.off_ws = off;
   off += align256((size_t)p.nchunk * H * E * sizeof(float));
   p.total = off;
@@ -2372,15 +2560,15 @@ void launch_dxdw_stream(hipStream_t s, const uint16_t* x, const uint16_t* wg, co
                         float* ws, uint16_t* g_out = nullptr, int g_pitch = 0, const uint16_t* dx_add = nullptr) {
   const char* name = dx ? "k_router_dxdw_bf16" : "k_router_dw_bf16";
 #define MOE_DXDW_STREAM(EL_, KR_, WPB_)                                                                               \
-  MOE_LAUNCH(name, (k_router_dxdw_stream<NTE, EL_, KR_, WPB_>), dim3((unsigned)(nchunk * (H / (64 * WPB_)))),          \
+  MOE_LAUNCH(name, (k_router_dxdw_stream<NTE, EL_, KR_, WPB_>), dim3((unsigned)(nchunk * cdiv(H, 64 * WPB_))),         \
              dim3(64 * WPB_), 0, s, x, wg, logits, idx, gw, gw_dt, cnt, grad_aux, grad_z, aux_coef, z_coef, N, H, E, K,  \
-             tc_len, H / (64 * WPB_), dx, dx_add, ws, g_out, g_pitch)
+             tc_len, cdiv(H, 64 * WPB_), dx, dx_add, ws, g_out, g_pitch)
   // G over 8 expert slots when E <= 8 (fewer registers while the first x tiles are in flight); the top-k
   // slots preloaded: 2 when K <= 2 (shorter code: the prologue runs on a cold instruction cache), else 4;
   // 16-wave blocks (1024 columns) when H allows
   if constexpr (NTE == 1) {
     if (E <= 8) {
-      if (H % 1024 == 0) {
+      if (H % 1024 == 0) {  // 16-wave blocks; else 4-wave blocks of 256 columns, the last one perhaps partial
         if (K <= 2) MOE_DXDW_STREAM(8, 2, 16);
         else MOE_DXDW_STREAM(8, kGRegK, 16);
       } else {
@@ -2403,7 +2591,7 @@ void launch_dxdw(dim3 grid, hipStream_t s, const uint16_t* x, const uint16_t* wg
 
 }  // namespace
 
-bool router_dw_g_applies(int64_t H, int64_t E) { return E <= 16 && H % 256 == 0; }
+bool router_dw_g_applies(int64_t H, int64_t E) { return E <= 16 && H % 8 == 0; }
 
 size_t router_dw_g_workspace(int64_t N, int64_t H, int64_t E) {
   const BwdPlan p = plan_bwd(N > 0 ? N : 1, H, E, MOE_BF16, MOE_BF16);
@@ -2440,7 +2628,11 @@ extern "C" int64_t moe_router_fwd_lds_bytes(int64_t N, int64_t H, int64_t E, int
   if (p.f32) {
     // the MFMA form when x is 16-byte aligned (the usual case); all TG variants share their LDS layout per NT
     f = p.NT == 1 ? (const void*)k_router_fwd_f32<1, 1> : p.NT == 2 ? (const void*)k_router_fwd_f32<2, 1>
-                                                                     : (const void*)k_router_fwd_f32<4, 1>;
+        : p.NT == 4 ? (const void*)k_router_fwd_f32<4, 1> : p.NT == 8 ? (const void*)k_router_fwd_f32<8, 1>
+                                                                       : (const void*)k_router_fwd_f32<16, 1>;
+  } else if (p.split) {
+    f = p.NT == 4 ? (const void*)k_router_fwd_split<4> : p.NT == 8 ? (const void*)k_router_fwd_split<8>
+                                                                  : (const void*)k_router_fwd_split<16>;
   } else if (p.wide) {
     f = p.NT == 4 ? (const void*)k_router_fwd_wide<4> : p.NT == 8 ? (const void*)k_router_fwd_wide<8>
                                                                  : (const void*)k_router_fwd_wide<16>;
@@ -2509,13 +2701,15 @@ extern "C" int moe_router_fwd(const void* x, int x_dtype, const void* wg, int wg
   } while (0)
     if (p.NT == 1) MOE_FWDF_TG(1);
     else if (p.NT == 2) MOE_FWDF_TG(2);
-    else MOE_FWDF_TG(4);
+    else if (p.NT == 4) MOE_FWDF_TG(4);
+    else if (p.NT == 8) MOE_FWDF_TG(8);
+    else MOE_FWDF_TG(16);
 #undef MOE_FWDF_TG
 #undef MOE_FWDF
     return check_launch("k_router_fwd_f32");
   }
   const bool mfma = p.mfma && aligned16(x);
-  if (mfma && p.stream) {
+  if (p.stream) {
     // streaming form: raw gate, finalize folded into the last block (ticket zero on entry and on exit)
     unsigned* ticket = reinterpret_cast<unsigned*>(ws + p.off_ticket);
     const uint16_t* xb = static_cast<const uint16_t*>(x);
@@ -2536,29 +2730,33 @@ extern "C" int moe_router_fwd(const void* x, int x_dtype, const void* wg, int wg
 #undef MOE_FWDS
     return check_launch("k_router_fwd_bf16");
   }
-  if (mfma && p.wide) {
+  const int gchunks = gate_chunks(H);
+  const int64_t glanes = (int64_t)gchunks * p.NT * 64;
+  if (p.wide) {
     // wide streaming form: packed gate, finalize folded into the last block (ticket zero on entry and on exit)
     i16x8* wp = reinterpret_cast<i16x8*>(ws + p.off_wp);
-    const int64_t lanes = (int64_t)(H / 32) * p.NT * 64;
-    MOE_LAUNCH("k_pack_gate", k_pack_gate, dim3((unsigned)std::min<int64_t>(1024, (lanes + 255) / 256)), dim3(256), 0, s,
-               static_cast<const uint16_t*>(wg), (int)H, (int)E, p.NT, wp, nullptr);
+    MOE_LAUNCH("k_pack_gate", k_pack_gate, dim3((unsigned)std::min<int64_t>(1024, (glanes + 255) / 256)), dim3(256), 0, s,
+               static_cast<const uint16_t*>(wg), (int)H, (int)E, p.NT, gchunks, wp);
     unsigned* ticket = reinterpret_cast<unsigned*>(ws + p.off_ticket);
     const uint16_t* xb = static_cast<const uint16_t*>(x);
-#define MOE_FWDW(NTv)                                                                                               \
-  MOE_LAUNCH("k_router_fwd_bf16", (k_router_fwd_wide<NTv>), dim3(p.nblk), dim3(512), 0, s, xb, wp, bias, (int)N,     \
+#define MOE_FWDW(KERNEL)                                                                                            \
+  MOE_LAUNCH("k_router_fwd_bf16", (KERNEL), dim3(p.nblk), dim3(512), 0, s, xb, wp, bias, (int)N,                     \
              (int)H, (int)E, (int)K, idx_out, w_out, w_dtype, logits_out, lse_out, pc, pp, pz, ticket, aux_coef,   \
              z_coef, cnt_out, stats_out, aux_out, z_out)
-    if (p.NT == 4) MOE_FWDW(4);
-    else if (p.NT == 8) MOE_FWDW(8);
-    else MOE_FWDW(16);
+    if (p.split) {
+      if (p.NT == 4) MOE_FWDW(k_router_fwd_split<4>);
+      else if (p.NT == 8) MOE_FWDW(k_router_fwd_split<8>);
+      else MOE_FWDW(k_router_fwd_split<16>);
+    } else if (p.NT == 4) MOE_FWDW(k_router_fwd_wide<4>);
+    else if (p.NT == 8) MOE_FWDW(k_router_fwd_wide<8>);
+    else MOE_FWDW(k_router_fwd_wide<16>);
 #undef MOE_FWDW
     return check_launch("k_router_fwd_bf16");
   }
   if (mfma) {
     i16x8* wp = reinterpret_cast<i16x8*>(ws + p.off_wp);
-    const int64_t lanes = (int64_t)((H + 31) / 32) * p.NT * 64;
-    MOE_LAUNCH("k_pack_gate", k_pack_gate, dim3((unsigned)std::min<int64_t>(1024, (lanes + 255) / 256)), dim3(256), 0, s,
-                       static_cast<const uint16_t*>(wg), (int)H, (int)E, p.NT, wp, nullptr);
+    MOE_LAUNCH("k_pack_gate", k_pack_gate, dim3((unsigned)std::min<int64_t>(1024, (glanes + 255) / 256)), dim3(256), 0, s,
+               static_cast<const uint16_t*>(wg), (int)H, (int)E, p.NT, gchunks, wp);
     const dim3 grid(p.nblk);
     const uint16_t* xb = static_cast<const uint16_t*>(x);
     switch (p.NT) {
@@ -2633,12 +2831,13 @@ extern "C" int moe_router_bwd_acc(const void* x, int x_dtype, const void* wg, in
   char* ws = static_cast<char*>(workspace);
   float* G = reinterpret_cast<float*>(ws + p.off_g);
   float* wsdw = reinterpret_cast<float*>(ws + p.off_ws);
-  const bool mfma = p.mfma && aligned16(x) && aligned16(dx_out);
-  uint16_t* gb = mfma ? reinterpret_cast<uint16_t*>(ws + p.off_gb) : nullptr;
+  const bool al = aligned16(x) && aligned16(dx_out);
+  const bool mfma = p.mfma && al;  // reached with an unaligned gate only
+  uint16_t* gb = al && p.wide ? reinterpret_cast<uint16_t*>(ws + p.off_gb) : nullptr;
   int nchunk = p.nchunk;
   const bool add_fused = dx_add != nullptr && x_dtype == MOE_BF16 && aligned16(dx_add);
   const uint16_t* addb = add_fused ? static_cast<const uint16_t*>(dx_add) : nullptr;
-  if (mfma && p.stream) {
+  if (al && p.stream) {
     // streaming form: dL/dlogits is formed inside the dx / dwg kernel, per chunk
     const uint16_t* xb = static_cast<const uint16_t*>(x);
     const uint16_t* wb = static_cast<const uint16_t*>(wg);
@@ -2654,7 +2853,7 @@ extern "C" int moe_router_bwd_acc(const void* x, int x_dtype, const void* wg, in
     launch_reduce(s, wsdw, nchunk, H * E, dwg_out, wg_dtype);
     return check_launch("moe_router_bwd");
   }
-  if (mfma && p.wide && aligned16(wg)) {
+  if (al && p.wide && aligned16(wg)) {
     // wide form: dL/dlogits in bf16 only (16 lanes per token), then the streaming dx / dwg kernel
     const int ekp = p.EK * 32;
 #define MOE_GLOGW(EPL)                                                                                         \
@@ -2669,7 +2868,7 @@ extern "C" int moe_router_bwd_acc(const void* x, int x_dtype, const void* wg, in
     const uint16_t* xb = static_cast<const uint16_t*>(x);
     const uint16_t* wb = static_cast<const uint16_t*>(wg);
     uint16_t* dxb = static_cast<uint16_t*>(dx_out);
-    const int nht = (int)(H / 256);
+    const int nht = cdiv(H, 256);
     const dim3 grid((unsigned)(p.nchunk * nht));
     if (p.EK == 2)
       MOE_LAUNCH("k_router_dxdw_bf16", (k_router_dxdw_wide<2, 4>), grid, dim3(256), 0, s, xb, wb, gb, (int)N, (int)H,
@@ -2705,9 +2904,7 @@ extern "C" int moe_router_bwd_acc(const void* x, int x_dtype, const void* wg, in
     uint16_t* dxb = static_cast<uint16_t*>(dx_out);
 #define MOE_DXDW(EKv, NTEv) \
   launch_dxdw<EKv, NTEv>(grid, s, xb, wb, gb, (int)N, (int)H, (int)E, p.tc_len, dxb, wsdw)
-    if (p.EK == 1 && p.NTE == 1) MOE_DXDW(1, 1);
-    else if (p.EK == 1 && p.NTE == 2) MOE_DXDW(1, 2);
-    else if (p.EK == 2 && p.NTE == 4) MOE_DXDW(2, 4);
+    if (p.EK == 2 && p.NTE == 4) MOE_DXDW(2, 4);
     else if (p.EK == 4 && p.NTE == 8) MOE_DXDW(4, 8);
     else return fail_arg("moe_router_bwd: internal tile error");
 #undef MOE_DXDW
@@ -2724,6 +2921,19 @@ extern "C" int moe_router_bwd_acc(const void* x, int x_dtype, const void* wg, in
       MOE_LAUNCH("k_router_dxdw_f32", k_router_dxdw_f32<16>, grid, dim3(256), 0, s, xf, wf, G, (int)N, (int)H, (int)E,
                  p.tc_len, dxf, wsdw);
     if (int rc = check_launch("k_router_dxdw_f32")) return rc;
+  } else if (p.f32m && aligned16(wg)) {
+    const float* xf = static_cast<const float*>(x);
+    MOE_LAUNCH("k_router_dx_f32", k_router_dx_f32, dim3((unsigned)cdiv(N, 64), (unsigned)cdiv(H, 64)), dim3(256), 0, s, G,
+               static_cast<const float*>(wg), (int)N, (int)H, (int)E, static_cast<float*>(dx_out));
+    const dim3 grid((unsigned)cdiv(H, 64), (unsigned)p.nchunk);
+#define MOE_DWF(NTEv) \
+  MOE_LAUNCH("k_router_dw_f32", k_router_dw_f32<NTEv>, grid, dim3(256), 0, s, xf, G, (int)N, (int)H, (int)E, p.tc_len, wsdw)
+    if (E <= 32) MOE_DWF(2);
+    else if (E <= 64) MOE_DWF(4);
+    else if (E <= 128) MOE_DWF(8);
+    else MOE_DWF(16);
+#undef MOE_DWF
+    if (int rc = check_launch("k_router_dw_f32")) return rc;
   } else {
     const int64_t NH = N * H;
     MOE_LAUNCH("k_router_dx_generic", k_router_dx_generic, dim3((unsigned)std::min<int64_t>(16384, (NH + 255) / 256)), dim3(256), 0,
