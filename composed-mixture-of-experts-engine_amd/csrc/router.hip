@@ -992,9 +992,11 @@ __global__ __launch_bounds__(512) void k_router_fwd_wide(
 // Forward for few tokens and many experts (bf16 x bf16, 32 < E <= 256, H % 8 == 0, N up to kSplitTokens).  The wide
 // form's 128-token blocks leave most CUs without one there and stream the whole hidden dim in turn; here a block is
 // one group of 16 tokens and its 8 waves take every 8th 32-column chunk of the hidden dim, with x and the packed gate
-// loaded straight into MFMA fragments.  The partial logit tiles are summed in LDS in wave order, and wave 0 routes.
-// Latency bound (a chain of H / 256 chunk loads a wave); the gate is re-read from L2 by every block, which is what
-// ends its use with more tokens.  H = 2048, E = 128, K = 8, 64 tokens: 36-43 us in the wide form, here 12 us.
+// loaded straight into MFMA fragments.  The partial logit tiles are summed in LDS in wave order, and each wave routes
+// two tokens with 32 lanes a token: the routing is a serial chain of K rounds, and one wave routing all 16 tokens
+// (route_quad: 4 lanes a token, E / 4 logits a lane) was half of the kernel's time.  The gate is re-read from L2 by
+// every block, which is what ends the form's use with more tokens.  H = 2048, E = 128, K = 8, 64 tokens: 36-43 us in
+// the wide form, 28 us with route_quad, 18 us here.
 // ---------------------------------------------------------------------------
 constexpr int kSplitTokens = 4096;
 
@@ -1005,19 +1007,25 @@ __global__ __launch_bounds__(512) void k_router_fwd_split(
     float* __restrict__ lse_out, int* __restrict__ part_cnt, float* __restrict__ part_p, float* __restrict__ part_z,
     unsigned* __restrict__ ticket, float aux_coef, float z_coef, int64_t* __restrict__ cnt_out,
     float* __restrict__ stats, float* __restrict__ aux_out, float* __restrict__ z_out) {
-  __shared__ f32x4 s_acc[7 * NT * 64];
-  __shared__ float s_tile[NT <= 8 ? 16 * (NT * 16 + 4) : 1];
+  constexpr int EL = NT / 2;       // logits a lane: experts l + 32 j
+  constexpr int LP = NT * 16 + 1;  // row pitch of the logit tile (floats)
+  __shared__ f32x4 s_acc[8 * NT * 64];
+  __shared__ float s_lg[16 * LP];
   __shared__ int s_cnt[NT * 16];
   __shared__ float s_p[1][NT * 16];
+  __shared__ float s_lse2[16];
   __shared__ float s_z[1];
   __shared__ int s_nf[1];
   __shared__ int s_last;
-  __shared__ float s_fin[finalize_scratch_floats<512>()];
+  static_assert(8 * NT * 64 * 4 >= finalize_scratch_floats<512>(), "the fold's scratch fits the partial tiles");
+  float* const s_fin = reinterpret_cast<float*>(s_acc);  // once the logits are formed
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, n = lane & 15;
   const int t0 = blockIdx.x * 16;
   for (int i = threadIdx.x; i < NT * 16; i += 512) s_cnt[i] = 0;
+  if (threadIdx.x < 16) s_lse2[threadIdx.x] = 0.f;
+  if (threadIdx.x == 0) s_nf[0] = 0;
 
   const uint16_t* const xr = x + (int64_t)min(t0 + n, N - 1) * H + g * 8;
   const i16x8* const wb = wp + lane;
@@ -1025,7 +1033,7 @@ __global__ __launch_bounds__(512) void k_router_fwd_split(
   f32x4 acc[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll(NT <= 4 ? 4 : NT == 8 ? 2 : 1)
+#pragma unroll(NT <= 8 ? 4 : 2)
   for (int c = wv; c < nc; c += 8) {
     // units past H: zeros (their gate rows are packed as zeros)
     const bool in = c * 32 + g * 8 < H;
@@ -1035,22 +1043,101 @@ __global__ __launch_bounds__(512) void k_router_fwd_split(
     for (int nt = 0; nt < NT; ++nt)
       acc[nt] = mfma16x16x32(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, wb[(c * NT + nt) * 64]), acc[nt]);
   }
-  if (wv > 0) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) s_acc[((wv - 1) * NT + nt) * 64 + lane] = acc[nt];
+  for (int nt = 0; nt < NT; ++nt) s_acc[(wv * NT + nt) * 64 + lane] = acc[nt];
+  __syncthreads();
+  // the block's 16 x E logits, summed in wave order: unit u holds tokens 4 (u / 16 % 4) + i of expert
+  // 16 (u / 64) + u % 16
+  int nf = 0;
+  for (int u = threadIdx.x; u < NT * 64; u += 512) {
+    f32x4 v = s_acc[u];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) v += s_acc[w * NT * 64 + u];
+    const int e = (u >> 6) * 16 + (u & 15), r0 = ((u >> 4) & 3) * 4;
+    if (bias != nullptr && e < E) v += bias[e];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float l = v[i];
+      if (t0 + r0 + i < N && e < E) {
+        logits_out[(int64_t)(t0 + r0 + i) * E + e] = l;
+        nf += isfinite(l) ? 0 : 1;
+      }
+      if (l != l || e >= E) l = -INFINITY;  // NaN (and experts past E) never win a top-k slot
+      s_lg[(r0 + i) * LP + e] = l;
+    }
+  }
+  if (nf) atomicAdd(&s_nf[0], nf);
+  __syncthreads();
+  {
+    const int r = 2 * wv + (lane >> 5), l = lane & 31, tt = t0 + r;
+    const bool valid = tt < N;
+    float lg[EL], ex[EL], m = -INFINITY, sum = 0.f;
+    uint32_t kh[EL];
+#pragma unroll
+    for (int j = 0; j < EL; ++j) {
+      lg[j] = s_lg[r * LP + l + 32 * j];
+      m = fmaxf(m, lg[j]);
+      kh[j] = l + 32 * j < E ? order_key(lg[j]) : 0u;
+    }
+    m = row16_max(m);
+    m = fmaxf(m, __shfl_xor(m, 16));
+#pragma unroll
+    for (int j = 0; j < EL; ++j) {
+      ex[j] = expf(lg[j] - m);
+      sum += ex[j];
+    }
+    sum = row16_sum(sum);
+    sum += __shfl_xor(sum, 16);
+    const float inv = 1.f / sum, lse = m + logf(sum);
+    if (valid && l == 0) {
+      lse_out[tt] = lse;
+      s_lse2[r] = lse * lse;
+    }
+    // K rounds of an arg-max over the keys; the lowest expert wins a tie; round k's pick is kept by lane k
+    int my_e = 0;
+    float my_p = 0.f, psum = 0.f;
+    for (int k = 0; k < K; ++k) {
+      uint32_t bh = kh[0];
+      int bj = 0;
+#pragma unroll
+      for (int j = 1; j < EL; ++j) {  // strict '>' keeps the lower expert
+        const bool t = kh[j] > bh;
+        bh = t ? kh[j] : bh;
+        bj = t ? j : bj;
+      }
+      int be = bh ? l + 32 * bj : 0x7fffffff;
+      uint32_t w = row16_max_u32(bh);
+      w = max(w, (uint32_t)__shfl_xor((int)w, 16));
+      be = row16_min_i32(bh == w ? be : 0x7fffffff);
+      be = min(be, __shfl_xor(be, 16));
+#pragma unroll
+      for (int j = 0; j < EL; ++j) kh[j] = l + 32 * j == be ? 0u : kh[j];
+      const float pv = expf(order_val(w) - m) * inv;
+      psum += pv;
+      my_e = k == l ? be : my_e;
+      my_p = k == l ? pv : my_p;
+    }
+    const float rden = 1.f / fmaxf(psum, 1e-30f);
+    if (valid && l < K) {
+      idx_out[(int64_t)tt * K + l] = my_e;
+      store_f(w_out, w_dt, (int64_t)tt * K + l, my_p * rden);
+      atomicAdd(&s_cnt[my_e], 1);
+    }
+#pragma unroll
+    for (int j = 0; j < EL; ++j) s_lg[r * LP + l + 32 * j] = valid ? ex[j] * inv : 0.f;
   }
   __syncthreads();
-  if (wv == 0) {
-#pragma unroll 1  // one wave's tiles at a time: all at once would not fit the registers
-    for (int w = 0; w < 7; ++w)
+  for (int e = threadIdx.x; e < NT * 16; e += 512) {  // probability sums, in token order
+    float p = 0.f;
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[nt] += s_acc[(w * NT + nt) * 64 + lane];
-    if constexpr (NT <= 8)
-      route_quad<NT>(acc, s_tile, t0, lane, bias, N, E, K, idx_out, w_out, w_dt, logits_out, lse_out, s_cnt, s_p[0],
-                     &s_z[0], &s_nf[0]);
-    else
-      route_group<NT>(acc, t0, lane, bias, N, E, K, idx_out, w_out, w_dt, logits_out, lse_out, s_cnt, s_p[0], &s_z[0],
-                      &s_nf[0]);
+    for (int r = 0; r < 16; ++r) p += s_lg[r * LP + e];
+    s_p[0][e] = p;
+  }
+  if (threadIdx.x == 0) {
+    float z = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) z += s_lse2[r];
+    s_z[0] = z;
   }
   __syncthreads();
   fwd_block_tail<1, NT>(s_cnt, s_p, s_z, s_nf, s_last, s_fin, N, E, K, part_cnt, part_p, part_z, ticket, aux_coef,
