@@ -475,7 +475,7 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
     for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
       for (int ni = 0; ni < NI; ++ni)
-        acc[mi][ni] = mfma32x32x16(__builtin_bit_cast(bf16x8, fa[mi]), __builtin_bit_cast(bf16x8, fb[ni]), acc[mi][ni]);
+        acc[mi][ni] = mfma32x32x16(__builtin_bit_cast(bf16x8, fb[ni]), __builtin_bit_cast(bf16x8, fa[mi]), acc[mi][ni]);
   };
 
   static_assert(!F8 || NW == 4, "the fp8 products run the 4-wave loop");
@@ -602,10 +602,10 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
              constexpr int i = SLO + I;
              constexpr int mi = i / NI, ni = i % NI;
              if constexpr (MX)
-               acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[mi], fb[ni], acc[mi][ni], 0, 0,
-                                                                             2 * ST, sw[mi], 0, 127);
+               acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[ni], fa[mi], acc[mi][ni], 0, 0, 0, 127,
+                                                                             2 * ST, sw[mi]);
              else
-               acc[mi][ni] = mfma32x32x64_f8(fa[mi], fb[ni], acc[mi][ni]);
+               acc[mi][ni] = mfma32x32x64_f8(fb[ni], fa[mi], acc[mi][ni]);
              __builtin_amdgcn_sched_barrier(0);
              if (read_next) {
                if constexpr (ni == NI - 1) fa[mi] = frag_rows_f8(nas, wm0 + mi * 32, nst, lane);
@@ -689,7 +689,7 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
         (([&] {
            constexpr int i = I;
            constexpr int mi = i / NI, ni = i % NI;
-           acc[mi][ni] = mfma32x32x16(__builtin_bit_cast(bf16x8, ca[mi]), __builtin_bit_cast(bf16x8, cb[ni]), acc[mi][ni]);
+           acc[mi][ni] = mfma32x32x16(__builtin_bit_cast(bf16x8, cb[ni]), __builtin_bit_cast(bf16x8, ca[mi]), acc[mi][ni]);
            __builtin_amdgcn_sched_barrier(0);
            if constexpr (i < MI + NI) {
              if (read_next) read_frag(nas, nbs, nks, i, na, nb);
@@ -808,8 +808,14 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
   }
   __syncthreads();
 
-  // ---- epilogue: the bf16 C tile goes through LDS so every global access is a 16-byte row chunk.
-  // acc[mi][ni][j] = C[wm0 + mi*32 + (j/4)*8 + (lane/32)*4 + j%4][wn0 + ni*32 + lane%32]
+  // ---- epilogue: the bf16 C tile goes through LDS so every global access is a 16-byte row chunk.  The MFMAs take the
+  // B fragment as their M operand, so a lane holds one C row and, in each four accumulators, four columns in a row:
+  // acc[mi][ni][j] = C[wm0 + mi*32 + lane%32][wn0 + ni*32 + (j/4)*8 + (lane/32)*4 + j%4]
+  // (8-byte LDS writes; with a column a lane and the rows in its accumulators they were 2-byte ones, four times as
+  // many: E = 128, H = 2048, F = 768 fwd2 787 -> 740 us; E = 8, H = 4096, F = 14336, 250 rows an expert, dWd and dW1
+  // 1360 -> 1288).
+  const int er = wm0 + (lane & 31);        // + 32 mi
+  const int ec = wn0 + (lane >> 5) * 4;    // + 32 ni + 8 (j / 4) + j % 4
   constexpr int CP = GCP;
   uint16_t* cs = reinterpret_cast<uint16_t*>(smem);
   if constexpr (F8) {
@@ -836,24 +842,31 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
         // the general path, reading one 16-byte act chunk instead of the gate and up chunks)
         constexpr int AP = GBN / 2 + 8;
         static_assert(NI == 4, "two gate/up pairs per wave");
-        // column scales of the lane's two pairs (gate, up); each row scale is read once for both pairs, and
-        // each bf16 rounding converts two values at once (the same rounding as one at a time)
-        const int cg0 = wn0 + (lane & 31), cg1 = cg0 + 64;
-        const float sg0 = s_sc[256 + cg0], su0 = s_sc[256 + cg0 + 32];
-        const float sg1 = s_sc[256 + cg1], su1 = s_sc[256 + cg1 + 32];
-        const int fc0 = (cg0 >> 6) * 32 + (lane & 31), fc1 = (cg1 >> 6) * 32 + (lane & 31);
+        // a lane's four columns of each 8: their scales are one 16-byte read, the row's scale is the lane's own
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
+        for (int pr = 0; pr < NI / 2; ++pr)
 #pragma unroll
-          for (int j = 0; j < 16; ++j) {
-            const int r = wm0 + mi * 32 + (j >> 2) * 8 + (lane >> 5) * 4 + (j & 3);
-            const float sr = s_sc[r];
-            const uint32_t gu0 = pack2bf(acc[mi][0][j] * sr * sg0, acc[mi][1][j] * sr * su0);
-            const uint32_t gu1 = pack2bf(acc[mi][2][j] * sr * sg1, acc[mi][3][j] * sr * su1);
-            const uint32_t a01 = pack2bf(silu_f(__uint_as_float(gu0 << 16)) * __uint_as_float(gu0 & 0xffff0000u),
-                                         silu_f(__uint_as_float(gu1 << 16)) * __uint_as_float(gu1 & 0xffff0000u));
-            cs[r * AP + fc0] = (uint16_t)a01;
-            cs[r * AP + fc1] = (uint16_t)(a01 >> 16);
+          for (int v = 0; v < 4; ++v) {
+            const int cg = ec + 2 * pr * 32 + v * 8;  // gate column; the up column is 32 on
+            const f32x4 sg = *reinterpret_cast<const f32x4*>(&s_sc[256 + cg]);
+            const f32x4 su = *reinterpret_cast<const f32x4*>(&s_sc[256 + cg + 32]);
+            const int fc = (cg >> 6) * 32 + (cg & 31);
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi) {
+              const int r = er + mi * 32;
+              const float sr = s_sc[r];
+              uint32_t o[2];
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const int j = 4 * v + 2 * h;
+                const uint32_t gq = pack2bf(acc[mi][2 * pr][j] * sr * sg[2 * h], acc[mi][2 * pr][j + 1] * sr * sg[2 * h + 1]);
+                const uint32_t uq =
+                    pack2bf(acc[mi][2 * pr + 1][j] * sr * su[2 * h], acc[mi][2 * pr + 1][j + 1] * sr * su[2 * h + 1]);
+                o[h] = pack2bf(silu_f(__uint_as_float(gq << 16)) * __uint_as_float(uq << 16),
+                               silu_f(__uint_as_float(gq & 0xffff0000u)) * __uint_as_float(uq & 0xffff0000u));
+              }
+              *reinterpret_cast<uint2*>(&cs[r * AP + fc]) = uint2{o[0], o[1]};
+            }
           }
         __syncthreads();
         constexpr int QPR = GBN / 16;  // 8-f chunks per row
@@ -892,15 +905,19 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
       }
     }
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
+    for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-      for (int ni = 0; ni < NI; ++ni) {
-        const int c = wn0 + ni * 32 + (lane & 31);
-        const float sc = s_sc[256 + c];
+      for (int v = 0; v < 4; ++v) {
+        const int c = ec + ni * 32 + v * 8;
+        const f32x4 sc = *reinterpret_cast<const f32x4*>(&s_sc[256 + c]);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int r = wm0 + mi * 32 + (j >> 2) * 8 + (lane >> 5) * 4 + (j & 3);
-          cs[r * CP + c] = f2bf(acc[mi][ni][j] * s_sc[r] * sc);
+        for (int mi = 0; mi < MI; ++mi) {
+          const int r = er + mi * 32;
+          const float sr = s_sc[r];
+          const f32x16& t = acc[mi][ni];
+          *reinterpret_cast<uint2*>(&cs[r * CP + c]) =
+              uint2{pack2bf(t[4 * v] * sr * sc[0], t[4 * v + 1] * sr * sc[1]),
+                    pack2bf(t[4 * v + 2] * sr * sc[2], t[4 * v + 3] * sr * sc[3])};
         }
       }
   } else {
@@ -913,17 +930,22 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-          for (int pr = 0; pr < NI / 2; ++pr) {
-            const int cg = wn0 + 2 * pr * 32 + (lane & 31);
-            const int fc = (cg >> 6) * 32 + (lane & 31);
+          for (int pr = 0; pr < NI / 2; ++pr)
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-              const int r = wm0 + mi * 32 + (j >> 2) * 8 + (lane >> 5) * 4 + (j & 3);
-              const float gq = __uint_as_float((uint32_t)f2bf(acc[mi][2 * pr][j]) << 16);
-              const float uq = __uint_as_float((uint32_t)f2bf(acc[mi][2 * pr + 1][j]) << 16);
-              cs[r * AP + fc] = f2bf(silu_f(gq) * uq);
+            for (int v = 0; v < 4; ++v) {
+              const int cg = ec + 2 * pr * 32 + v * 8;
+              const int fc = (cg >> 6) * 32 + (cg & 31);
+              uint32_t o[2];
+#pragma unroll
+              for (int h = 0; h < 2; ++h) {
+                const int j = 4 * v + 2 * h;
+                const uint32_t gq = pack2bf(acc[mi][2 * pr][j], acc[mi][2 * pr][j + 1]);
+                const uint32_t uq = pack2bf(acc[mi][2 * pr + 1][j], acc[mi][2 * pr + 1][j + 1]);
+                o[h] = pack2bf(silu_f(__uint_as_float(gq << 16)) * __uint_as_float(uq << 16),
+                               silu_f(__uint_as_float(gq & 0xffff0000u)) * __uint_as_float(uq & 0xffff0000u));
+              }
+              *reinterpret_cast<uint2*>(&cs[(er + mi * 32) * AP + fc]) = uint2{o[0], o[1]};
             }
-          }
         __syncthreads();
         constexpr int QPR = GBN / 16;  // 8-f chunks per row
         for (int u = tid; u < GBM * QPR; u += GNT) {
@@ -941,9 +963,10 @@ __global__ __launch_bounds__(NW * 64, 1) void k_gemm(GemmArgs g) {
 #pragma unroll
       for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int r = wm0 + mi * 32 + (j >> 2) * 8 + (lane >> 5) * 4 + (j & 3);
-          cs[r * CP + wn0 + ni * 32 + (lane & 31)] = f2bf(acc[mi][ni][j]);
+        for (int v = 0; v < 4; ++v) {
+          const f32x16& t = acc[mi][ni];
+          *reinterpret_cast<uint2*>(&cs[(er + mi * 32) * CP + ec + ni * 32 + v * 8]) =
+              uint2{pack2bf(t[4 * v], t[4 * v + 1]), pack2bf(t[4 * v + 2], t[4 * v + 3])};
         }
   }
   __syncthreads();
@@ -1116,23 +1139,36 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(GemmArgs g) {
   const int mbase = g.offsets[e] + mt * GBM, mlen = min(GBM, g.offsets[e + 1] - mbase);
   const f32x4* const src = reinterpret_cast<const f32x4*>(g.part + (int64_t)(xcd * g.npart + t * S) * (GBM * GBN));
   constexpr int U = GBM * GBN / 4;  // 16-byte units of a tile
-  for (int u = (int)blockIdx.y * (U / 8) + threadIdx.x; u < (int)(blockIdx.y + 1) * (U / 8); u += 256) {
-    // unit: wave, (mi, ni), v, lane, as k_gemm stores them
-    const int lane = u & 63, v = (u >> 6) & 3, blk = (u >> 8) % (MI * NI), wv = (u >> 8) / (MI * NI);
-    const int r0 = (wv / NW_N) * GWM + (blk / NI) * 32 + v * 8 + (lane >> 5) * 4;
-    const int c = nt * GBN + (wv % NW_N) * (NI * 32) + (blk % NI) * 32 + (lane & 31);
-    if (r0 >= mlen || c >= g.N) continue;
+  // 256 units are one 32x32 block, as k_gemm stores them: (wave, (mi, ni)), v, lane; it goes through LDS so that its
+  // rows leave as 64-byte segments
+  constexpr int BP = 36;  // block pitch (bf16): 8-byte writes, rows 18 banks apart
+  __shared__ __attribute__((aligned(16))) uint16_t blkt[2][32 * BP];
+  const int lane = threadIdx.x & 63, v = threadIdx.x >> 6;
+  int buf = 0;
+  for (int b = (int)blockIdx.y * (U / 2048); b < (int)(blockIdx.y + 1) * (U / 2048); ++b) {
+    const int blk = b % (MI * NI), wv = b / (MI * NI);
+    const int rb = (wv / NW_N) * GWM + (blk / NI) * 32, cb = nt * GBN + (wv % NW_N) * (NI * 32) + (blk % NI) * 32;
+    if (rb >= mlen || cb >= g.N) continue;  // the same for the whole block
+    const int u = b * 256 + threadIdx.x;
     f32x4 s = src[u];
     for (int p = 1; p < S; ++p) s += src[(int64_t)p * U + u];
-    const float sc = g.sb != nullptr ? g.sb[(int64_t)e * g.N + c] : 1.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (r0 + j < mlen) g.C[(int64_t)(mbase + r0 + j) * g.ldc + c] = f2bf(s[j] * sc);
+    const int c = v * 8 + (lane >> 5) * 4;
+    if (g.sb != nullptr && cb + c < g.N) {  // N % 8 == 0
+      const float* const sb = g.sb + (int64_t)e * g.N + cb + c;
+      s *= f32x4{sb[0], sb[1], sb[2], sb[3]};
+    }
+    *reinterpret_cast<uint2*>(&blkt[buf][(lane & 31) * BP + c]) = uint2{pack2bf(s[0], s[1]), pack2bf(s[2], s[3])};
+    __syncthreads();  // between a buffer's readers and its next writers lies the other buffer's barrier
+    const int r = threadIdx.x >> 3, q = (threadIdx.x & 7) * 4;
+    if (rb + r < mlen && cb + q < g.N)
+      *reinterpret_cast<uint2*>(g.C + (int64_t)(mbase + rb + r) * g.ldc + cb + q) =
+          *reinterpret_cast<const uint2*>(&blkt[buf][r * BP + q]);
+    buf ^= 1;  // only where a block was moved: a skipped one has no barrier
   }
 }
 
-// tile_off[0] = 0, tile_off[e+1] = sum_{e' <= e} ceil(rows_e' / bm)  (one block, E <= 1024), and the
-// expert order of the k-grouped products: experts ranked by rows (descending, lower id first on a tie) are
+// tile_off[0] = 0, tile_off[e+1] = sum_{e' <= e} ceil(rows_e' / bm)  (one block, E <= 1024), and, with
+// korder, the expert order of the k-grouped products: experts ranked by rows (descending, lower id first on a tie) are
 // dealt to the 8 XCD ranges in snake order (rank r -> range r % 8 on even rounds, 7 - r % 8 on odd ones),
 // and korder lists range 0's experts by rank, then range 1's, ...
 __global__ __launch_bounds__(1024) void k_gemm_tiles(const int* __restrict__ offsets, int E, int bm,
@@ -1148,14 +1184,14 @@ __global__ __launch_bounds__(1024) void k_gemm_tiles(const int* __restrict__ off
   if (tid < 8) xcnt[tid] = 0;
   __syncthreads();
   int rank = 0, x = 0, j = 0;
-  if (tid < E) {
+  if (korder != nullptr && tid < E) {
     for (int f = 0; f < E; ++f) rank += (rows[f] > nrow || (rows[f] == nrow && f < tid)) ? 1 : 0;
     j = rank >> 3;
     x = (j & 1) ? 7 - (rank & 7) : (rank & 7);
     atomicAdd(&xcnt[x], 1);
   }
   __syncthreads();
-  if (tid == 0) {
+  if (korder != nullptr && tid == 0) {
     int b = 0;
     for (int q = 0; q < 8; ++q) {
       xbase[q] = b;
@@ -1163,8 +1199,8 @@ __global__ __launch_bounds__(1024) void k_gemm_tiles(const int* __restrict__ off
     }
   }
   __syncthreads();
-  if (tid < E) korder[xbase[x] + j] = tid;
-  for (int o = 1; o < 1024; o <<= 1) {
+  if (korder != nullptr && tid < E) korder[xbase[x] + j] = tid;
+  for (int o = 1; o < E; o <<= 1) {
     const int v = tid >= o ? part[tid - o] : 0;
     __syncthreads();
     part[tid] += v;
@@ -1177,6 +1213,11 @@ __global__ __launch_bounds__(1024) void k_gemm_tiles(const int* __restrict__ off
 namespace {
 bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 unsigned round8(int64_t v) { return (unsigned)((v + 7) / 8 * 8); }
+
+void launch_tiles(hipStream_t s, const int* offsets, int64_t E, int* tile_off, int* korder) {
+  const unsigned threads = (unsigned)((E + 63) / 64 * 64);
+  MOE_LAUNCH("k_gemm_tiles", k_gemm_tiles, dim3(1), dim3(threads), 0, s, offsets, (int)E, GBM, tile_off, korder);
+}
 
 template <int AM, int BMD, int GR, int EP, int NW>
 int launch(const char* name, hipStream_t s, const GemmArgs& a, int64_t R) {
@@ -1221,7 +1262,6 @@ void take_split(GemmArgs& a, int64_t R, void* ws, size_t ws_bytes, size_t used) 
   a.npart = split_parts(R, a.E, a.N);
 }
 
-constexpr int kTileBM = GBM;
 // Wave layout per product: 4 waves of 128x128 (one per SIMD; register-staged refill two slices ahead) for the
 // forward products (bf16 and fp8), whose operands are both k-contiguous; 8 waves of 128x64 (LDS-DMA refill)
 // for the backward products.  The row-grouped tile prefix is computed with the kernels' BM.
@@ -1252,8 +1292,7 @@ extern "C" int moe_swiglu_fwd(const void* xp, const void* w_gate, const void* w_
   if (swiglu_small_takes(R, H, F, E, 2))
     return swiglu_small_fwd(false, xp, w_gate, w_up, w_down, offsets, R, H, F, E, act, hgu, y, s);
   int* tile_off = static_cast<int*>(workspace);
-  int* korder = tile_off + (E + 1);
-  MOE_LAUNCH("k_gemm_tiles", k_gemm_tiles, dim3(1), dim3(1024), 0, s, offsets, (int)E, kTileBM, tile_off, korder);
+  launch_tiles(s, offsets, E, tile_off, nullptr);
   GemmArgs a{};
   a.offsets = offsets;
   a.tile_off = tile_off;
@@ -1324,10 +1363,9 @@ extern "C" int moe_swiglu_fwd_fp8(const void* xq, const float* sx, const void* w
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
   int* tile_off = reinterpret_cast<int*>(ws);
-  int* korder = tile_off + (E + 1);
   uint8_t* actq = reinterpret_cast<uint8_t*>(ws + moe_swiglu_workspace(E));
   uint8_t* sact = reinterpret_cast<uint8_t*>(ws + moe_swiglu_workspace(E) + fp8_act_bytes(R, F));
-  MOE_LAUNCH("k_gemm_tiles", k_gemm_tiles, dim3(1), dim3(1024), 0, s, offsets, (int)E, kTileBM, tile_off, korder);
+  launch_tiles(s, offsets, E, tile_off, nullptr);
   // fwd1: [act | hgu] = (xq sx) . ([Wg ; Wu] [sg ; su])^T; fp8 matrices are addressed in 16-bit units
   GemmArgs a{};
   a.offsets = offsets;
@@ -1388,7 +1426,7 @@ extern "C" int moe_swiglu_bwd(const void* dy, const void* xp, const void* act, c
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   int* tile_off = static_cast<int*>(workspace);
   int* korder = tile_off + (E + 1);
-  MOE_LAUNCH("k_gemm_tiles", k_gemm_tiles, dim3(1), dim3(1024), 0, s, offsets, (int)E, kTileBM, tile_off, korder);
+  launch_tiles(s, offsets, E, tile_off, korder);
   // dA: dh = epilogue(dy . Wd)   (B[n=f][k=h] = Wd[h][f])
   if (R > 0) {
     GemmArgs a{};
