@@ -59,6 +59,7 @@ _SIGNATURES = {
     "moe_permute": (_I32, [_P, _I64, _P, _P, _I64, _I64, _I64, _P, _P]),
     "moe_combine": (_I32, [_P, _I32, _P, _I32, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P]),
     "moe_combine_bwd": (_I32, [_P, _P, _I32, _P, _I32, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _P]),
+    "moe_zero_tail": (_I32, [_P, _I64, _P, _I64, _I64, _P]),
     "moe_unpermute_sum": (_I32, [_P, _P, _I32, _P, _P, _I64, _I64, _I64, _I64, _P, _P]),
     "moe_rmsnorm_fwd": (_I32, [_P, _I32, _P, _I32, _F32, _I64, _I64, _P, _P, _P]),
     "moe_rmsnorm_router_fwd_workspace": (_SZ, [_I64, _I64, _I64, _I64, _I32, _I32]),

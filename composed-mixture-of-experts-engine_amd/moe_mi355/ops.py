@@ -406,17 +406,21 @@ def combine(y: torch.Tensor, w: torch.Tensor, p: Plan) -> torch.Tensor:
 def combine_backward(dout: torch.Tensor, y: torch.Tensor, w: torch.Tensor, p: Plan, need_dw: bool = True,
                      zero_tail: bool = False):
     """Returns (dy [rows, H], dw [N, K] or None).  Rows past offsets[E] of dy are
-    left unwritten unless ``zero_tail`` (then the whole buffer starts at zero)."""
+    left unwritten unless ``zero_tail`` (then they are zeros)."""
     dev = L.require_device(dout, y, w)
     dout = dout.contiguous()
     H = y.shape[1]
-    dy = torch.zeros_like(y) if zero_tail else torch.empty_like(y)
+    dy = torch.empty_like(y)
     dw = torch.empty((p.N, p.K), dtype=w.dtype, device=dev) if need_dw else None
     rc = L.load().moe_combine_bwd(dout.data_ptr(), y.data_ptr(), L.dtype_code(y.dtype), w.contiguous().data_ptr(),
                                   L.dtype_code(w.dtype), L.ptr(p.drop_u8()), p.slot_row.data_ptr(),
                                   p.offsets.data_ptr(), p.N, p.K, H, p.E, dy.data_ptr(), L.ptr(dw),
                                   L.stream_of(dev))
     L.check(rc, "moe_combine_bwd")
+    if zero_tail:
+        rc = L.load().moe_zero_tail(dy.data_ptr(), H * dy.element_size(), p.offsets.data_ptr(), p.E, dy.shape[0],
+                                    L.stream_of(dev))
+        L.check(rc, "moe_zero_tail")
     return dy, dw
 
 

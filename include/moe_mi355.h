@@ -227,6 +227,9 @@ int moe_combine(const void* y, int dtype, const void* w, int w_dtype, const uint
 int moe_combine_bwd(const void* dout, const void* y, int dtype, const void* w, int w_dtype, const uint8_t* drop,
                     const int32_t* slot_row, const int32_t* offsets, int64_t N, int64_t K, int64_t H, int64_t E,
                     void* dy, void* dw, void* stream);
+/* Zeros in the rows [offsets[E], rows) of a buffer of row_bytes (a multiple of 16) rows: those that moe_combine_bwd
+ * leaves unwritten. */
+int moe_zero_tail(void* y, int64_t row_bytes, const int32_t* offsets, int64_t E, int64_t rows, void* stream);
 
 /* Permute backward: dx[t] = addend[t] (NULL = 0) + sum_k dxp[slot_row[t*K+k]]
  * over computed rows.  The autograd backward of L:318-319. */
