@@ -129,6 +129,24 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The native binding (moe_mi355/_moe_torch.so, built with libmoe_mi355.so)."""
+    global _native
+    if _native is None:
+        try:
+            from . import _moe_torch
+        except ImportError as e:
+            raise RuntimeError(
+                "moe_mi355/_moe_torch.so is not built or does not load; run __graft_entry__.build() "
+                f"(or python moe_mi355/build.py) on a host with ROCm/hipcc ({e})"
+            ) from e
+        _native = _moe_torch
+    return _native
+
+
 def last_error() -> str:
     buf = ctypes.create_string_buffer(512)
     load().moe_last_error(buf, 512)
@@ -216,36 +234,6 @@ def stream_of(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-_ws_cache = {}
-_ARENA_BYTES = 32 << 20
-_capture_arena = {}  # device index -> [zeroed buffer, bytes handed out]
-
-
-def workspace(nbytes: int, device: torch.device, key: Optional[str] = None) -> torch.Tensor:
-    """Scratch memory for one call.  With ``key``, a workspace that must start zeroed and that the kernels
-    leave zeroed where it matters (the router forward's ticket counter): one zero-initialised buffer per
-    (key, device, stream), reused by every call on that stream (stream order serialises them).  Under
-    graph capture each capture takes a fresh slice of a per-device arena zeroed (and synchronised) once
-    outside any capture, so the graph holds no fill node (a zeroed buffer made inside the capture once the
-    arena is used up)."""
-    n = max(int(nbytes), 1)
-    if key is None:
-        return torch.empty(n, dtype=torch.uint8, device=device)
-    arena = _capture_arena.get(device.index)
-    if torch.cuda.is_current_stream_capturing():
-        n256 = (n + 255) // 256 * 256
-        if arena is not None and arena[1] + n256 <= _ARENA_BYTES:
-            buf = arena[0].narrow(0, arena[1], n)
-            arena[1] += n256
-            return buf
-        return torch.zeros(n, dtype=torch.uint8, device=device)
-    if arena is None:
-        _capture_arena[device.index] = [torch.zeros(_ARENA_BYTES, dtype=torch.uint8, device=device), 0]
-        torch.cuda.current_stream(device).synchronize()  # once: later captures may replay on any stream
-    stream = torch.cuda.current_stream(device).cuda_stream
-    k = (key, device.index, stream)
-    buf = _ws_cache.get(k)
-    if buf is None or buf.numel() < n:
-        buf = torch.zeros(n, dtype=torch.uint8, device=device)
-        _ws_cache[k] = buf
-    return buf
+def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
+    """Scratch memory for one call."""
+    return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)

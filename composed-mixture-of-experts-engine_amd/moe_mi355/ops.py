@@ -1,5 +1,6 @@
-"""Tensor-level wrappers over the C ABI: allocate outputs with torch's caching
-allocator, pass raw pointers and the current stream, check the return code.
+"""Tensor-level wrappers over the C ABI: outputs from torch's caching allocator, raw pointers and the current
+stream, the return code checked.  What a layer's pass runs goes through the native binding (csrc/torch_router.cpp),
+the rest through ctypes.
 
 No function here synchronises the host or falls back to a CPU path.
 """
@@ -35,8 +36,6 @@ def router_forward(
     ``with_losses``; the stats layout is documented in include/moe_mi355.h.
     """
     dev = L.require_device(x, gate_w, bias)
-    x = x.contiguous()
-    gate_w = gate_w.contiguous()
     N, H = x.shape
     H2, E = gate_w.shape
     if H != H2:
@@ -44,36 +43,20 @@ def router_forward(
     w_dtype = w_dtype or x.dtype
     if bias is not None:
         bias = bias.detach().to(torch.float32).contiguous()
-    lib = L.load()
-    xdt, wdt, odt = L.dtype_code(x.dtype), L.dtype_code(gate_w.dtype), L.dtype_code(w_dtype)
-    idx = torch.empty((N, k), dtype=torch.int64, device=dev)
-    w = torch.empty((N, k), dtype=w_dtype, device=dev)
-    logits = torch.empty((N, E), dtype=torch.float32, device=dev)
-    lse = torch.empty((N,), dtype=torch.float32, device=dev)
-    cnt = torch.empty((E,), dtype=torch.int64, device=dev)
-    stats = torch.empty((L.STATS_HEAD + E,), dtype=torch.float32, device=dev)
-    aux = torch.empty((), dtype=torch.float32, device=dev) if with_losses else None
-    z = torch.empty((), dtype=torch.float32, device=dev) if with_losses else None
+    L.dtype_code(x.dtype), L.dtype_code(gate_w.dtype)
+    w_bf16 = L.dtype_code(w_dtype) == L.MOE_BF16
     if N == 0:
-        cnt.zero_()
-        stats.zero_()
-        if with_losses:
-            aux.zero_()
-            z.zero_()
-            return idx, w, logits, lse, cnt, stats, aux, z
-        return idx, w, logits, lse, cnt, stats
-    nbytes = lib.moe_router_fwd_workspace(N, H, E, k, xdt, wdt)
-    ws = L.workspace(nbytes, dev, key="router_fwd")  # zeroed once; the kernel leaves its ticket at zero
-    rc = lib.moe_router_fwd(
-        x.data_ptr(), xdt, gate_w.data_ptr(), wdt, L.ptr(bias), N, H, E, k,
-        idx.data_ptr(), w.data_ptr(), odt, logits.data_ptr(), lse.data_ptr(),
-        cnt.data_ptr(), stats.data_ptr(), float(aux_coef), float(z_coef), L.ptr(aux), L.ptr(z),
-        ws.data_ptr(), nbytes, L.stream_of(dev),
-    )
-    L.check(rc, "moe_router_fwd")
-    if with_losses:
-        return idx, w, logits, lse, cnt, stats, aux, z
-    return idx, w, logits, lse, cnt, stats
+        idx = torch.empty((N, k), dtype=torch.int64, device=dev)
+        w = torch.empty((N, k), dtype=w_dtype, device=dev)
+        logits = torch.empty((N, E), dtype=torch.float32, device=dev)
+        lse = torch.empty((N,), dtype=torch.float32, device=dev)
+        cnt = torch.zeros((E,), dtype=torch.int64, device=dev)
+        stats = torch.zeros((L.STATS_HEAD + E,), dtype=torch.float32, device=dev)
+        aux, z = torch.zeros((), dtype=torch.float32, device=dev), torch.zeros((), dtype=torch.float32, device=dev)
+        out = (idx, w, logits, lse, cnt, stats, aux, z)
+    else:
+        out = tuple(L.native().router_forward(x, gate_w, int(k), bias, w_bf16, float(aux_coef), float(z_coef)))
+    return out if with_losses else out[:6]
 
 
 def router_backward(
@@ -184,32 +167,16 @@ def rmsnorm_router_forward(
         raise ValueError(f"rmsnorm_router_forward: hidden dims differ ({H} vs {H2})")
     if bias is not None:
         bias = bias.detach().to(torch.float32).contiguous()
-    lib = L.load()
-    xdt, gdt, wdt = L.dtype_code(x.dtype), L.dtype_code(weight.dtype), L.dtype_code(gate_w.dtype)
-    xn = torch.empty_like(x)
-    rstd = torch.empty((N,), dtype=torch.float32, device=dev)
-    idx = torch.empty((N, k), dtype=torch.int64, device=dev)
-    w = torch.empty((N, k), dtype=x.dtype, device=dev)
-    logits = torch.empty((N, E), dtype=torch.float32, device=dev)
-    lse = torch.empty((N,), dtype=torch.float32, device=dev)
-    cnt = torch.empty((E,), dtype=torch.int64, device=dev)
-    stats = torch.empty((L.STATS_HEAD + E,), dtype=torch.float32, device=dev)
-    aux = torch.empty((), dtype=torch.float32, device=dev)
-    z = torch.empty((), dtype=torch.float32, device=dev)
+    for t in (x, weight, gate_w):
+        L.dtype_code(t.dtype)
     if N == 0:
-        for t in (cnt, stats, aux, z):
-            t.zero_()
-        return xn, rstd, idx, w, logits, lse, cnt, stats, aux, z
-    nbytes = lib.moe_rmsnorm_router_fwd_workspace(N, H, E, k, xdt, wdt)
-    ws = L.workspace(nbytes, dev, key="router_fwd")  # zeroed once; the kernels leave the counter at zero
-    rc = lib.moe_rmsnorm_router_fwd(
-        x.data_ptr(), xdt, weight.data_ptr(), gdt, float(eps), gate_w.data_ptr(), wdt, L.ptr(bias), N, H, E, k,
-        xn.data_ptr(), rstd.data_ptr(), idx.data_ptr(), w.data_ptr(), xdt, logits.data_ptr(), lse.data_ptr(),
-        cnt.data_ptr(), stats.data_ptr(), float(aux_coef), float(z_coef), aux.data_ptr(), z.data_ptr(),
-        ws.data_ptr(), nbytes, L.stream_of(dev),
-    )
-    L.check(rc, "moe_rmsnorm_router_fwd")
-    return xn, rstd, idx, w, logits, lse, cnt, stats, aux, z
+        f32 = dict(dtype=torch.float32, device=dev)
+        return (torch.empty_like(x), torch.empty((N,), **f32), torch.empty((N, k), dtype=torch.int64, device=dev),
+                torch.empty((N, k), dtype=x.dtype, device=dev), torch.empty((N, E), **f32), torch.empty((N,), **f32),
+                torch.zeros((E,), dtype=torch.int64, device=dev), torch.zeros((L.STATS_HEAD + E,), **f32),
+                torch.zeros((), **f32), torch.zeros((), **f32))
+    return tuple(L.native().rmsnorm_router_forward(x, weight, float(eps), gate_w, int(k), bias, float(aux_coef),
+                                                   float(z_coef)))
 
 
 def rmsnorm_backward(
@@ -261,43 +228,22 @@ def rmsnorm_router_backward(
     :func:`router_backward`) and a gradient ``dxn`` of ``xn`` from the expert path (or None).
 
     Returns ``(dx [N,H] x.dtype, dweight [H] weight.dtype, dgate_w [H,E] gate_w.dtype)``."""
-    dev = L.require_device(x, weight, rstd, xn, gate_w, logits, idx, grad_w, dxn, cnt)
-    x = x.contiguous()
-    weight = weight.contiguous()
-    xn = xn.contiguous()
-    gate_w = gate_w.contiguous()
-    logits = logits.contiguous()
-    idx = idx.contiguous()
+    L.require_device(x, weight, rstd, xn, gate_w, logits, idx, grad_w, dxn, cnt)
+    _, _ = x.shape
+    for t in (x, weight, gate_w):
+        L.dtype_code(t.dtype)
     if dxn is not None:
         dxn = dxn.contiguous().to(x.dtype)
-    N, H = x.shape
-    E = gate_w.shape[1]
-    K = idx.shape[1]
-    lib = L.load()
-    xdt, ndt, wdt = L.dtype_code(x.dtype), L.dtype_code(weight.dtype), L.dtype_code(gate_w.dtype)
-    gdt = L.MOE_F32
     if grad_w is not None:
         grad_w = grad_w.contiguous()
         if grad_w.dtype not in (torch.float32, torch.bfloat16):
             grad_w = grad_w.float()
-        gdt = L.dtype_code(grad_w.dtype)
     if grad_aux is not None:
         grad_aux = grad_aux.detach().to(torch.float32).reshape(1).contiguous()
     if grad_z is not None:
         grad_z = grad_z.detach().to(torch.float32).reshape(1).contiguous()
-    dx = torch.empty_like(x)
-    dweight = torch.empty_like(weight)
-    dgate = torch.empty((H, E), dtype=gate_w.dtype, device=dev)
-    nbytes = lib.moe_rmsnorm_router_bwd_workspace(N, H, E, K, xdt, wdt)
-    ws = L.workspace(nbytes, dev)
-    rc = lib.moe_rmsnorm_router_bwd(
-        x.data_ptr(), xdt, weight.data_ptr(), ndt, rstd.data_ptr(), xn.data_ptr(), gate_w.data_ptr(), wdt,
-        logits.data_ptr(), idx.data_ptr(), L.ptr(grad_w), gdt, L.ptr(cnt), L.ptr(grad_aux), L.ptr(grad_z),
-        float(aux_coef), float(z_coef), L.ptr(dxn), N, H, E, K, dx.data_ptr(), dweight.data_ptr(),
-        dgate.data_ptr(), ws.data_ptr(), nbytes, L.stream_of(dev),
-    )
-    L.check(rc, "moe_rmsnorm_router_bwd")
-    return dx, dweight, dgate
+    return tuple(L.native().rmsnorm_router_backward(x, weight, rstd, xn, gate_w, logits, idx, grad_w, dxn, cnt, grad_aux,
+                                                    grad_z, float(aux_coef), float(z_coef)))
 
 
 # ---------------------------------------------------------------------------
@@ -351,19 +297,18 @@ def cumcount(groups: torch.Tensor) -> torch.Tensor:
 def plan(idx: torch.Tensor, num_experts: int, capacity: int = -1, layout: int = LAYOUT_REFERENCE) -> Plan:
     """Build the dispatch plan from the router's top-k indices (no host sync)."""
     dev = L.require_device(idx)
-    idx = idx.contiguous()
-    if idx.dtype != torch.int64:
-        idx = idx.long()
     N, K = idx.shape
     E = int(num_experts)
+    M = N * K
+    if M > 0:
+        return Plan(*L.native().plan(idx, E, int(capacity), int(layout)), N, K, E, layout)
+    idx = idx.contiguous().long()
     lib = L.load()
     drop = torch.empty((N, K), dtype=torch.bool, device=dev) if capacity >= 0 else None
-    M = N * K
-    row_slot = torch.empty((max(M, 1),), dtype=torch.int32, device=dev)
-    slot_row = torch.empty((max(M, 1),), dtype=torch.int32, device=dev)
+    row_slot = torch.empty((1,), dtype=torch.int32, device=dev)
+    slot_row = torch.empty((1,), dtype=torch.int32, device=dev)
     offsets = torch.empty((E + 1,), dtype=torch.int32, device=dev)
-    ndrop = torch.zeros((1,), dtype=torch.int32, device=dev) if M == 0 else torch.empty((1,), dtype=torch.int32,
-                                                                                         device=dev)
+    ndrop = torch.zeros((1,), dtype=torch.int32, device=dev)
     nbytes = lib.moe_plan_workspace(N, K, E)
     ws = L.workspace(nbytes, dev)
     rc = lib.moe_plan(
@@ -379,62 +324,31 @@ def permute(x: torch.Tensor, p: Plan) -> torch.Tensor:
     """xp [N*K, H]: row slot_row[t*K+k] holds x[t] (one read of each token row; rows past offsets[E] are left
     unwritten)."""
     dev = L.require_device(x)
-    x = x.contiguous()
-    H = x.shape[1]
-    xp = torch.empty((p.rows, H), dtype=x.dtype, device=dev)
     if p.rows == 0:
-        return xp
-    rc = L.load().moe_permute(x.data_ptr(), H * x.element_size(), p.slot_row.data_ptr(), p.offsets.data_ptr(),
-                              p.N, p.K, p.E, xp.data_ptr(), L.stream_of(dev))
-    L.check(rc, "moe_permute")
-    return xp
+        return torch.empty((0, x.shape[1]), dtype=x.dtype, device=dev)
+    return L.native().permute(x, p.slot_row, p.offsets, p.N, p.K, p.E)
 
 
 def combine(y: torch.Tensor, w: torch.Tensor, p: Plan) -> torch.Tensor:
-    dev = L.require_device(y, w)
-    y = y.contiguous()
-    w = w.contiguous()
-    H = y.shape[1]
-    out = torch.empty((p.N, H), dtype=y.dtype, device=dev)
-    rc = L.load().moe_combine(y.data_ptr(), L.dtype_code(y.dtype), w.data_ptr(), L.dtype_code(w.dtype),
-                              L.ptr(p.drop_u8()), p.slot_row.data_ptr(), p.offsets.data_ptr(), p.N, p.K, H, p.E,
-                              out.data_ptr(), L.stream_of(dev))
-    L.check(rc, "moe_combine")
-    return out
+    L.require_device(y, w)
+    L.dtype_code(y.dtype), L.dtype_code(w.dtype)
+    return L.native().combine(y, w, p.drop, p.slot_row, p.offsets, p.N, p.K, p.E)
 
 
 def combine_backward(dout: torch.Tensor, y: torch.Tensor, w: torch.Tensor, p: Plan, need_dw: bool = True,
                      zero_tail: bool = False):
     """Returns (dy [rows, H], dw [N, K] or None).  Rows past offsets[E] of dy are
     left unwritten unless ``zero_tail`` (then they are zeros)."""
-    dev = L.require_device(dout, y, w)
-    dout = dout.contiguous()
-    H = y.shape[1]
-    dy = torch.empty_like(y)
-    dw = torch.empty((p.N, p.K), dtype=w.dtype, device=dev) if need_dw else None
-    rc = L.load().moe_combine_bwd(dout.data_ptr(), y.data_ptr(), L.dtype_code(y.dtype), w.contiguous().data_ptr(),
-                                  L.dtype_code(w.dtype), L.ptr(p.drop_u8()), p.slot_row.data_ptr(),
-                                  p.offsets.data_ptr(), p.N, p.K, H, p.E, dy.data_ptr(), L.ptr(dw),
-                                  L.stream_of(dev))
-    L.check(rc, "moe_combine_bwd")
-    if zero_tail:
-        rc = L.load().moe_zero_tail(dy.data_ptr(), H * dy.element_size(), p.offsets.data_ptr(), p.E, dy.shape[0],
-                                    L.stream_of(dev))
-        L.check(rc, "moe_zero_tail")
-    return dy, dw
+    L.require_device(dout, y, w)
+    L.dtype_code(y.dtype), L.dtype_code(w.dtype)
+    return L.native().combine_backward(dout, y, w, p.drop, p.slot_row, p.offsets, p.N, p.K, p.E, bool(need_dw),
+                                       bool(zero_tail))
 
 
 def unpermute_sum(dxp: torch.Tensor, p: Plan, addend: Optional[torch.Tensor] = None) -> torch.Tensor:
-    dev = L.require_device(dxp, addend)
-    H = dxp.shape[1]
-    dx = torch.empty((p.N, H), dtype=dxp.dtype, device=dev)
-    if addend is not None:
-        addend = addend.contiguous()
-    rc = L.load().moe_unpermute_sum(dxp.contiguous().data_ptr(), L.ptr(addend), L.dtype_code(dxp.dtype),
-                                    p.slot_row.data_ptr(), p.offsets.data_ptr(), p.N, p.K, H, p.E, dx.data_ptr(),
-                                    L.stream_of(dev))
-    L.check(rc, "moe_unpermute_sum")
-    return dx
+    L.require_device(dxp, addend)
+    L.dtype_code(dxp.dtype)
+    return L.native().unpermute_sum(dxp, addend, p.slot_row, p.offsets, p.N, p.K, p.E)
 
 
 # ---------------------------------------------------------------------------
@@ -444,28 +358,11 @@ def swiglu_forward(xp: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w
                    offsets: torch.Tensor, keep_preact: bool = True):
     """xp [R,H]; w_gate/w_up [E,F,H]; w_down [E,H,F] (all bf16 or all fp32, contiguous) -> (act [R,F], hgu [R,2F],
     y [R,H]).  ``keep_preact=False`` (no backward follows) skips storing the pre-activations: hgu is None."""
-    dev = L.require_device(xp, w_gate, w_up, w_down, offsets)
-    f32 = _gemm_dtype_is_f32("swiglu_forward", xp, w_gate, w_up, w_down)
-    R, H = xp.shape
-    E, F, _ = w_gate.shape
-    act = torch.empty((R, F), dtype=xp.dtype, device=dev)
-    hgu = torch.empty((R, 2 * F), dtype=xp.dtype, device=dev) if keep_preact else None
-    y = torch.empty((R, H), dtype=xp.dtype, device=dev)
-    lib = L.load()
-    nbytes = _gemm_workspace(lib, f32, R, H, F, E)
-    ws = L.workspace(nbytes, dev)
-    fn = lib.moe_swiglu_fwd_f32 if f32 else lib.moe_swiglu_fwd
-    rc = fn(xp.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), w_down.data_ptr(), offsets.data_ptr(), R, H, F, E,
-            act.data_ptr(), L.ptr(hgu), y.data_ptr(), ws.data_ptr(), nbytes, L.stream_of(dev))
-    L.check(rc, "moe_swiglu_fwd_f32" if f32 else "moe_swiglu_fwd")
-    return act, hgu, y
-
-
-def _gemm_workspace(lib, f32: bool, R: int, H: int, F: int, E: int) -> int:
-    """Bytes of the grouped GEMM's tile tables and of the partial tiles of products split over k."""
-    if f32:
-        return lib.moe_swiglu_f32_workspace(E) + lib.moe_swiglu_f32_split_workspace(R, H, F, E)
-    return lib.moe_swiglu_workspace(E) + lib.moe_swiglu_split_workspace(R, H, F, E)
+    L.require_device(xp, w_gate, w_up, w_down, offsets)
+    _gemm_dtype_is_f32("swiglu_forward", xp, w_gate, w_up, w_down)
+    _, _ = xp.shape
+    _, _, _ = w_gate.shape
+    return L.native().swiglu_forward(xp, w_gate, w_up, w_down, offsets, bool(keep_preact))
 
 
 def _gemm_dtype_is_f32(what, *ts) -> bool:
@@ -559,22 +456,9 @@ def swiglu_forward_fp8(xq, sx, wq, wscale, offsets, out_dtype=torch.bfloat16, ke
 
 def swiglu_backward(dy, xp, act, hgu, w_gate, w_up, w_down, offsets):
     """-> (dxp [R,H], dw_gate [E,F,H], dw_up [E,F,H], dw_down [E,H,F])."""
-    dev = L.require_device(dy, xp, act, hgu, w_gate, w_up, w_down, offsets)
+    L.require_device(dy, xp, act, hgu, w_gate, w_up, w_down, offsets)
     dy = dy.contiguous()
-    f32 = _gemm_dtype_is_f32("swiglu_backward", dy, xp, act, hgu, w_gate, w_up, w_down)
-    R, H = xp.shape
-    E, F, _ = w_gate.shape
-    dh = torch.empty((R, 2 * F), dtype=xp.dtype, device=dev)
-    dxp = torch.empty((R, H), dtype=xp.dtype, device=dev)
-    dwg = torch.empty_like(w_gate)
-    dwu = torch.empty_like(w_up)
-    dwd = torch.empty_like(w_down)
-    lib = L.load()
-    nbytes = _gemm_workspace(lib, f32, R, H, F, E)
-    ws = L.workspace(nbytes, dev)
-    fn = lib.moe_swiglu_bwd_f32 if f32 else lib.moe_swiglu_bwd
-    rc = fn(dy.data_ptr(), xp.data_ptr(), act.data_ptr(), hgu.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(),
-            w_down.data_ptr(), offsets.data_ptr(), R, H, F, E, dh.data_ptr(), dxp.data_ptr(), dwg.data_ptr(),
-            dwu.data_ptr(), dwd.data_ptr(), ws.data_ptr(), nbytes, L.stream_of(dev))
-    L.check(rc, "moe_swiglu_bwd_f32" if f32 else "moe_swiglu_bwd")
-    return dxp, dwg, dwu, dwd
+    _gemm_dtype_is_f32("swiglu_backward", dy, xp, act, hgu, w_gate, w_up, w_down)
+    _, _ = xp.shape
+    _, _, _ = w_gate.shape
+    return tuple(L.native().swiglu_backward(dy, xp, act, hgu, w_gate, w_up, w_down, offsets))

@@ -34,22 +34,7 @@ STAT_NONFINITE = 6
 STAT_DEAD = 7
 
 
-_native = None
-
-
-def _binding():
-    """The native autograd binding (moe_mi355/_moe_torch.so, built with libmoe_mi355.so)."""
-    global _native
-    if _native is None:
-        try:
-            from . import _moe_torch
-        except ImportError as e:
-            raise RuntimeError(
-                "moe_mi355/_moe_torch.so is not built or does not load; run __graft_entry__.build() "
-                f"(or python moe_mi355/build.py) on a host with ROCm/hipcc ({e})"
-            ) from e
-        _native = _moe_torch
-    return _native
+_binding = L.native
 
 
 class RouterCore:
@@ -76,7 +61,7 @@ class RouterCore:
             raise ValueError(f"router_forward: hidden dims differ ({H} vs {H2})")
         L.dtype_code(x.dtype)
         L.dtype_code(gate_w.dtype)
-        return tuple(_binding().router_core(x, gate_w, int(k), float(aux_coef), float(z_coef), bias, bool(link_x)))
+        return tuple(L.native().router_core(x, gate_w, int(k), float(aux_coef), float(z_coef), bias, bool(link_x)))
 
 
 def route(x: torch.Tensor, gate_w: torch.Tensor, k: int, aux_coef: float = 0.0, z_coef: float = 0.0,
