@@ -12,7 +12,7 @@
 // An MFMA may take its two k values from any positions as long as A and B agree: in MFMA s of a group of 8 k, lane l
 // supplies k = 8 grp + 4 (l / 32) + s for its row (A) or column (B), so the four MFMAs of a group cover its 8 k once
 // each.  LDS holds an operand tile in its own order, so neither is transposed on the way in:
-//   operand mode 0 ("rows"): element (i, k) at P[i*ld + k]: [i][k] with a pitch of 20 floats; a lane reads the four k
+//   operand mode 0 ("rows"): element (i, k) at P[i*ld + k]: [i][k] with a pitch of 36 floats; a lane reads the four k
 //                            of a group with one 16-byte read
 //   operand mode 1 ("cols"): element (i, k) at P[k*ld + i]: [k][i] with a pitch of 136 floats; a lane reads its k's
 //                            one by one (4 bytes; the half waves are 4 rows = 32 banks apart, so no two lanes meet)
@@ -55,7 +55,7 @@ constexpr int FBM = 128, FBN = 128, FBK = 32;
 constexpr int FNT = 512;                 // threads: eight waves, two on each SIMD
 constexpr int FNJ = FBM * FBK / (4 * FNT);  // 16-byte units of an operand slice a thread moves
 constexpr int FCH = FBK / 4;           // ... and of one row of it
-constexpr int FKP = FBK + 4;    // rows mode: LDS row pitch (floats): 80 bytes, keeps 16-byte reads aligned
+constexpr int FKP = FBK + 4;    // rows mode: LDS row pitch (floats): 144 bytes, keeps 16-byte reads aligned
 constexpr int FIP = FBM + 8;    // cols mode: pitch of a k row (floats); 4 pitches are 32 banks mod 64
 constexpr int fop(int mode) { return mode ? FBK * FIP : FBM * FKP; }  // floats of an operand tile
 

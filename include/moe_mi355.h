@@ -340,7 +340,7 @@ int moe_swiglu_fwd_fp8(const void* xq, const float* sx, const void* wg_q, const 
  * backward of moe_router_bwd over xn (same grad_w / grad_aux / grad_z / cnt
  * contract; dwg_out in wg's dtype) and the norm backward of dxn plus the
  * router's gradient of xn (dxn may be null: no gradient from the expert path).
- * For bf16 x and gate with E <= 16 and H % 256 == 0 the router's gradient of
+ * For bf16 x and gate with E <= 16 the router's gradient of
  * xn is formed inside the norm kernel from dL/dlogits and never reaches HBM;
  * otherwise moe_router_bwd writes it to the workspace and moe_rmsnorm_bwd
  * adds it.
