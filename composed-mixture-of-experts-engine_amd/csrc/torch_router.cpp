@@ -49,13 +49,21 @@ using torch::autograd::variable_list;
 int code_of(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 ? MOE_BF16 : MOE_F32; }
 
 // The forward's workspace holds a ticket counter that must be zero when a launch starts and that the kernels
-// leave at zero: one zero-initialised buffer per (device, stream), reused by every call on that stream (stream
-// order serialises them).  Under graph capture each capture takes a fresh slice of a per-device arena instead,
+// leave at zero: one zero-initialised buffer per (device, stream), reused by every call on that stream.  A call
+// may launch several kernels that hand data on through it (the packed gate, the per-block partials), so stream
+// order keeps calls apart only if no other thread's launches come between one call's: FwdWorkspace holds the
+// buffer's lock until the call's last launch is queued (no call of this file holds the GIL meanwhile, so a
+// waiting thread stops no other).
+// Under graph capture each capture takes a fresh slice of a per-device arena instead,
 // zeroed and synchronised once outside any capture (on the first eager call): the kernels leave the counter at
 // zero after every replay, so that slice serves every replay of its graph, and the graph holds no fill node.
 // Captures past the arena's end fall back to a zeroed buffer made inside the capture (a captured fill kernel).
-std::mutex g_ws_mu;
-std::map<std::pair<int, hipStream_t>, at::Tensor> g_ws;
+struct StreamBuffer {
+  std::mutex mu;
+  at::Tensor buf;
+};
+std::mutex g_ws_mu;  // the two maps and the arenas; never held while a StreamBuffer's lock is waited for
+std::map<std::pair<int, hipStream_t>, StreamBuffer> g_ws;  // entries stay where they are (a map's nodes)
 constexpr int64_t kArenaBytes = 32 << 20;
 struct CaptureArena {
   at::Tensor buf;
@@ -63,36 +71,49 @@ struct CaptureArena {
 };
 std::map<int, CaptureArena> g_arena;
 
-at::Tensor fwd_workspace(size_t nbytes, const at::Device& dev, hipStream_t s) {
-  const int64_t n = std::max<int64_t>((int64_t)nbytes, 1);
-  const auto opts = at::TensorOptions().dtype(at::kByte).device(dev);
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-    (void)hipGetLastError();
-    throw std::runtime_error("moe_router_fwd: hipStreamIsCapturing failed");
-  }
-  std::lock_guard<std::mutex> lk(g_ws_mu);
-  CaptureArena& ar = g_arena[(int)dev.index()];
-  if (st != hipStreamCaptureStatusNone) {
-    const int64_t n256 = (n + 255) / 256 * 256;
-    if (ar.buf.defined() && ar.used + n256 <= kArenaBytes) {
-      at::Tensor slice = ar.buf.narrow(0, ar.used, n);
-      ar.used += n256;
-      return slice;
-    }
-    return at::zeros({n}, opts);
-  }
-  if (!ar.buf.defined()) {
-    ar.buf = at::zeros({kArenaBytes}, opts);
-    if (hipStreamSynchronize(s) != hipSuccess) {  // once: later captures may replay on any stream
+class FwdWorkspace {
+ public:
+  FwdWorkspace(size_t nbytes, const at::Device& dev, hipStream_t s) {
+    const int64_t n = std::max<int64_t>((int64_t)nbytes, 1);
+    const auto opts = at::TensorOptions().dtype(at::kByte).device(dev);
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
       (void)hipGetLastError();
-      throw std::runtime_error("moe_router_fwd: hipStreamSynchronize failed");
+      throw std::runtime_error("moe_router_fwd: hipStreamIsCapturing failed");
     }
+    StreamBuffer* sb = nullptr;
+    {
+      std::lock_guard<std::mutex> lk(g_ws_mu);
+      CaptureArena& ar = g_arena[(int)dev.index()];
+      if (st != hipStreamCaptureStatusNone) {
+        const int64_t n256 = (n + 255) / 256 * 256;
+        if (ar.buf.defined() && ar.used + n256 <= kArenaBytes) {
+          buf_ = ar.buf.narrow(0, ar.used, n);
+          ar.used += n256;
+        } else {
+          buf_ = at::zeros({n}, opts);
+        }
+        return;
+      }
+      if (!ar.buf.defined()) {
+        ar.buf = at::zeros({kArenaBytes}, opts);
+        if (hipStreamSynchronize(s) != hipSuccess) {  // once: later captures may replay on any stream
+          (void)hipGetLastError();
+          throw std::runtime_error("moe_router_fwd: hipStreamSynchronize failed");
+        }
+      }
+      sb = &g_ws[{(int)dev.index(), s}];
+    }
+    lock_ = std::unique_lock<std::mutex>(sb->mu);
+    if (!sb->buf.defined() || sb->buf.numel() < n) sb->buf = at::zeros({n}, opts);
+    buf_ = sb->buf;
   }
-  auto& buf = g_ws[{(int)dev.index(), s}];
-  if (!buf.defined() || buf.numel() < n) buf = at::zeros({n}, opts);
-  return buf;
-}
+  void* data_ptr() const { return buf_.data_ptr(); }
+
+ private:
+  at::Tensor buf_;
+  std::unique_lock<std::mutex> lock_;
+};
 
 struct RouterFn : public torch::autograd::Function<RouterFn> {
   // link_x: x is also returned, as an eighth output, for the layer's expert path to consume.  Its gradient
@@ -126,7 +147,7 @@ struct RouterFn : public torch::autograd::Function<RouterFn> {
       const hipStream_t s = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream();
       const int xdt = code_of(x), wdt = code_of(gw);
       const size_t nbytes = moe_router_fwd_workspace(N, H, E, k, xdt, wdt);
-      const at::Tensor ws = fwd_workspace(nbytes, dev, s);
+      const FwdWorkspace ws(nbytes, dev, s);
       const int rc = moe_router_fwd(x.data_ptr(), xdt, gw.data_ptr(), wdt,
                                     bias.defined() ? bias.data_ptr<float>() : nullptr, N, H, E, k,
                                     idx.data_ptr<int64_t>(), w.data_ptr(), xdt, logits.data_ptr<float>(),
@@ -231,7 +252,7 @@ std::vector<at::Tensor> op_router_forward(const at::Tensor& x_in, const at::Tens
   const hipStream_t s = stream_of(x);
   const int xdt = code_of(x), wdt = code_of(gw);
   const size_t nbytes = moe_router_fwd_workspace(N, H, E, k, xdt, wdt);
-  const at::Tensor ws = fwd_workspace(nbytes, x.device(), s);
+  const FwdWorkspace ws(nbytes, x.device(), s);
   check_rc(moe_router_fwd(x.data_ptr(), xdt, gw.data_ptr(), wdt, static_cast<const float*>(ptr(bias)), N, H, E, k,
                           idx.data_ptr<int64_t>(), w.data_ptr(), w_bf16 ? MOE_BF16 : MOE_F32, logits.data_ptr<float>(),
                           lse.data_ptr<float>(), cnt.data_ptr<int64_t>(), stats.data_ptr<float>(), (float)aux_coef,
@@ -255,7 +276,7 @@ std::vector<at::Tensor> op_rmsnorm_router_forward(const at::Tensor& x_in, const 
   const hipStream_t s = stream_of(x);
   const int xdt = code_of(x), wdt = code_of(gw);
   const size_t nbytes = moe_rmsnorm_router_fwd_workspace(N, H, E, k, xdt, wdt);
-  const at::Tensor ws = fwd_workspace(nbytes, x.device(), s);
+  const FwdWorkspace ws(nbytes, x.device(), s);
   check_rc(moe_rmsnorm_router_fwd(x.data_ptr(), xdt, weight.data_ptr(), code_of(weight), (float)eps, gw.data_ptr(), wdt,
                                   static_cast<const float*>(ptr(bias)), N, H, E, k, xn.data_ptr(), rstd.data_ptr<float>(),
                                   idx.data_ptr<int64_t>(), w.data_ptr(), xdt, logits.data_ptr<float>(),

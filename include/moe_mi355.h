@@ -105,7 +105,9 @@ int moe_prof_hbm_ceiling(int64_t bytes, int mode, double* gbps);
  * Workspace: zero it before its first use and reuse it for later calls on
  * the same stream.  Its first word is a completion counter that the call
  * expects at zero and leaves at zero (no other part of the library writes
- * it); calls that share a workspace must not overlap.
+ * it); calls that share a workspace must not overlap: the kernels of one
+ * call hand data on through it, so a call from another host thread may
+ * not queue its launches between them.
  * ---------------------------------------------------------------------- */
 size_t moe_router_fwd_workspace(int64_t N, int64_t H, int64_t E, int64_t K, int x_dtype, int wg_dtype);
 /* LDS bytes per workgroup of the forward kernel a call with these sizes and dtypes launches (-1 if the runtime
