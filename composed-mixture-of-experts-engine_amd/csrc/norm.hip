@@ -190,12 +190,13 @@ __device__ __forceinline__ float wave_reduce_scatter(const float (&acc)[NV], int
 //            h = 8 (l + 64 j) + 2 m, q < EP / 4
 //   backward (pairs along e): word ((q NCH + j) 8 + i) 64 + l, dword k = (wg[h][8q+2k], wg[h][8q+2k+1]),
 //            h = 8 (l + 64 j) + i, q < EP / 8
-// With E == EP (16-byte aligned rows) each gate row is read as EP / 8 16-byte words.
+// With E == EP and a 16-byte aligned gate (the backward takes any) each gate row is read as EP / 8 16-byte words.
 template <int EP>
 __device__ __forceinline__ void gate_row(const uint16_t* __restrict__ wg, int h, int H, int E, u32x4 (&r)[EP / 8]) {
+  const bool vec = E == EP && (reinterpret_cast<uintptr_t>(wg) & 15u) == 0;
 #pragma unroll
   for (int u = 0; u < EP / 8; ++u) {
-    if (E == EP) {
+    if (vec) {
       r[u] = h < H ? *reinterpret_cast<const u32x4*>(wg + (int64_t)h * EP + 8 * u) : u32x4{0u, 0u, 0u, 0u};
     } else {
 #pragma unroll

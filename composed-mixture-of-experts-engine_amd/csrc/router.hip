@@ -1924,7 +1924,9 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(NTE ==
 
   // gate fragments for dx: B[k = e][n = h] = wg[h][e]
   i16x8 wB[4];
-  if (E == 8) {  // each gate row is one 16-byte piece (lanes past the first 8 experts hold zeros)
+  // each gate row is one 16-byte piece (lanes past the first 8 experts hold zeros), unless the gate is a view that
+  // starts off such a boundary: only x and dx choose this kernel
+  if (E == 8 && (reinterpret_cast<uintptr_t>(wg) & 15u) == 0) {
 #pragma unroll
     for (int nc = 0; nc < 4; ++nc) {
       const i16x8 v = *reinterpret_cast<const i16x8*>(wg + (int64_t)min(col0 + nc * 16 + n, H - 1) * 8);

@@ -83,3 +83,30 @@ def test_unaligned_gate_and_tokens():
         assert torch.equal(a[0], b[0])
         # 64 x 96 products: fp32 sums in another order
         assert float((a[2] - b[2]).abs().max()) <= 2 * H * 2.0**-24 * float((x.abs().float() @ w.abs().float()).max())
+
+
+@pytest.mark.parametrize("H,E,K", [(264, 8, 2), (512, 8, 2), (1024, 8, 2), (264, 16, 4), (264, 5, 2), (96, 64, 4),
+                                   (520, 128, 4)])
+def test_unaligned_gate_backward(H, E, K):
+    """A gate that starts off a 16-byte boundary: the router's and the norm-fused backward read it by element (E = 8, 16)
+    or take the kernels that do.  The same bits where the same kernel runs; 32 < E: other kernels, whose dL/dlogits and
+    results may each round the other way to bf16 (2^-8 of a value)."""
+    N = 70
+    x, w, gw = base._inputs(N, H, E, K, B, B, seed=11)
+    ws = torch.empty(H * E + 8, dtype=B, device=dev())[1:1 + H * E].view(H, E).copy_(w)
+    assert ws.data_ptr() % 16 == 2 and ws.is_contiguous()
+    x, w, gw = x.to(dev()), w.to(dev()), gw.to(dev())
+    idx, _, logits = ops.router_forward(x, w, K)[:3]
+    a = ops.router_backward(x, w, logits, idx, gw)
+    b = ops.router_backward(x, ws, logits, idx, gw)
+    if E <= 32:
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    else:
+        for p, q in zip(a, b):
+            assert float((p.double() - q.double()).norm()) <= 2.0**-7 * float(p.double().norm())
+    if E <= 16:
+        nw, dxn = torch.ones(H, device=dev()), torch.randn(N, H, device=dev()).to(B)
+        xn, rstd, idx, _, logits = ops.rmsnorm_router_forward(x, nw, 1e-5, w, K)[:5]
+        a = ops.rmsnorm_router_backward(x, nw, rstd, xn, w, logits, idx, gw, dxn)
+        b = ops.rmsnorm_router_backward(x, nw, rstd, xn, ws, logits, idx, gw, dxn)
+        assert all(torch.equal(p, q) for p, q in zip(a, b))
