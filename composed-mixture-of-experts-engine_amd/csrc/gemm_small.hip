@@ -14,8 +14,10 @@
 // are a pass of their own blocks over its weights, so a skewed routing's passes run beside each other.  No tile table:
 // a block finds its rows from `offsets`.
 //
-// Blocks start their chunks at different columns (a hash of the block id, wrapping around the row): rows lie a power
-// of two apart, and blocks that walk them in step ask the same few memory channels.  Measured at E = 8, H = 4096,
+// Blocks start their chunks at different columns (a hash of the expert and its column tile, wrapping around the row):
+// rows lie a power of two apart, and blocks that walk them in step ask the same few memory channels.  The start decides
+// the order of a row's sums, so it depends on nothing else: a row has the same bits whatever other experts' rows, and its
+// own expert's, are beside it.  (The passes of a tile over the same weights walk them together.)  Measured at E = 8, H = 4096,
 // F = 14336, one row an expert: 591 us for both products in step, 487 us started apart (5.8 TB/s of weights, the
 // rate of a plain read stream here); 718 / 558 us with non-temporal loads (each 128-byte line is asked for in two
 // halves, which a cached load fetches once).  Against the 256-row tiles: 795 us; E = 128, H = 2048, F = 768: 319 ->
@@ -59,15 +61,15 @@ __device__ __forceinline__ f32x4 mma16(const u32x4& w, const u32x4& a, f32x4 c) 
   }
 }
 
-// One pass: rows [row0, row0 + min(rows, 16 MT)) of the segment against the block's 64 weight rows.
+// One pass: rows [row0, row0 + min(rows, 16 MT)) of the segment against the block's 16 NF weight rows.
 template <bool F32, bool GU, int NF, int NW, int MT>
 __device__ __forceinline__ void small_pass(const SmallArgs& g, const uint8_t* base0, const uint8_t* base1, int64_t row0,
-                                           int rows, int n0, float* red) {
+                                           int rows, int n0, uint32_t tile, float* red) {
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
   const uint32_t kb = g.kbytes;
   constexpr int RP = NF * 16 + 4;  // floats a row of the partial sums
-  // fragment f of the 64 weight rows: GU: 0, 1 gate rows, 2, 3 up rows; rows past N repeat the last one
+  // fragment f of the 16 NF weight rows: GU: the first NF / 2 gate rows, the others up rows; rows past N repeat the last
   uint32_t wo[NF], ao[MT];
 #pragma unroll
   for (int f = 0; f < NF; ++f) {
@@ -134,7 +136,7 @@ __device__ __forceinline__ void small_pass(const SmallArgs& g, const uint8_t* ba
         for (int m = 0; m < MT; ++m) acc[f][m] = mma16<F32>(wb[b][f][s], ab[AB == 2 ? b : 0][m][s], acc[f][m]);
   };
   const int nc = (int)((kb + 127) / 128);
-  const int start = (int)__umulhi(blockIdx.x * 0x9E3779B1u, (uint32_t)nc);
+  const int start = (int)__umulhi(tile * 0x9E3779B1u, (uint32_t)nc);
   auto at = [&](int i) {
     const int c = i + start;
     return c < nc ? c : c - nc;
@@ -251,8 +253,9 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void k_gemm_small(SmallArgs g) {
   const int n0 = nt * NF * (GU ? 8 : 16);
   const uint8_t* const b0 = g.B + (int64_t)e * g.b_ebytes;
   const uint8_t* const b1 = GU ? g.B2 + (int64_t)e * g.b_ebytes : nullptr;
-  if (hi - m0 > 16) small_pass<F32, GU, NF, NW, 2>(g, b0, b1, m0, min(32, hi - m0), n0, red);
-  else small_pass<F32, GU, NF, NW, 1>(g, b0, b1, m0, hi - m0, n0, red);
+  const uint32_t tile = (uint32_t)(e * g.Tn + nt);
+  if (hi - m0 > 16) small_pass<F32, GU, NF, NW, 2>(g, b0, b1, m0, min(32, hi - m0), n0, tile, red);
+  else small_pass<F32, GU, NF, NW, 1>(g, b0, b1, m0, hi - m0, n0, tile, red);
 }
 
 // 64 weight rows and four waves a block; where that leaves fewer than 512 blocks (two a CU), 32 rows and eight

@@ -66,3 +66,31 @@ def test_few_rows(case):
         yy = got @ d.t()  # the down projection of the act it was given
         dy = u * yy.abs() + (Fd + 4) * u32 * (got.abs() @ d.abs().t()) + 1e-30
         assert bool(((y[lo:hi].cpu().double() - yy).abs() <= dy).all())
+
+
+@pytest.mark.parametrize("name,H,Fd", [("bf16", 1032, 2080), ("f32", 516, 1056)])
+def test_rows_do_not_depend_on_their_neighbours(name, H, Fd):
+    """An expert's rows have the same bits whatever the other experts' rows are, and wherever in the expert's own rows
+    they lie: the first, a later and a partial 32-row pass, with passes of other experts ahead of them or none."""
+    say(f"[swiglu small] neighbours {name} H={H} F={Fd}")
+    dt = torch.bfloat16 if name == "bf16" else torch.float32
+    E = 12
+    g = torch.Generator().manual_seed(H)
+    wg, wu = ((torch.randn(E, Fd, H, generator=g) / H**0.5).to(dt).to(dev()) for _ in range(2))
+    wd = (torch.randn(E, H, Fd, generator=g) / Fd**0.5).to(dt).to(dev())
+    rows = torch.randn(70, H, generator=g).to(dt).to(dev())  # expert 7's
+
+    def run(before, own, after):
+        counts = [0] * E
+        counts[2], counts[7], counts[9] = before, own.shape[0], after
+        assert sum(counts) <= 16 * E
+        other = torch.randn(before + after, H, device=dev()).to(dt)
+        xp = torch.cat([other[:before], own, other[before:]])
+        offs = torch.tensor([0] + counts).cumsum(0).int().to(dev())
+        return [t[before:before + own.shape[0]] for t in ops.swiglu_forward(xp, wg, wu, wd, offs)]
+
+    want = run(0, rows, 0)
+    for before, after in ((65, 0), (100, 20), (1, 33)):
+        assert all(torch.equal(a, b) for a, b in zip(run(before, rows, after), want))
+    part = run(40, rows[37:], 3)  # the same rows as others of the segment
+    assert all(torch.equal(a, b[37:]) for a, b in zip(part, want))
