@@ -10,19 +10,27 @@
 // 64-byte half chunk of row r, and the four lanes of a row make one 64-byte request.  The k slot a value lands in
 // is free as long as both operands agree.  Each wave keeps one whole chunk of weights in flight beyond the one it
 // multiplies.  The tokens' fragments come from L2 (re-read by every block).  The waves' partial sums meet in LDS
-// in wave order (fp32), where the SwiGLU is formed with the large kernels' own roundings.  Every 32 rows of an expert
-// are a pass of their own blocks over its weights, so a skewed routing's passes run beside each other.  No tile table:
-// a block finds its rows from `offsets`.
+// in wave order (fp32), where the SwiGLU is formed with the large kernels' own roundings.  Every 64 rows of an
+// expert (fp32: 32) are a pass of their own blocks over its weights, so a skewed routing's passes run beside each other.
+// No tile table: a block finds its rows from `offsets`.
 //
 // Blocks start their chunks at different columns (a hash of the expert and its column tile, wrapping around the row):
 // rows lie a power of two apart, and blocks that walk them in step ask the same few memory channels.  The start decides
 // the order of a row's sums, so it depends on nothing else: a row has the same bits whatever other experts' rows, and its
-// own expert's, are beside it.  (The passes of a tile over the same weights walk them together.)  Measured at E = 8, H = 4096,
-// F = 14336, one row an expert: 591 us for both products in step, 487 us started apart (5.8 TB/s of weights, the
-// rate of a plain read stream here); 718 / 558 us with non-temporal loads (each 128-byte line is asked for in two
-// halves, which a cached load fetches once).  Against the 256-row tiles: 795 us; E = 128, H = 2048, F = 768: 319 ->
-// 210 us; fp32 E = 8, H = 1024, F = 4096: 463 -> 77 us (128-row tiles).  At 16 rows an expert 528 against 750 us,
-// at 24 597 against 750, at 32 637 against 749, at 64 (two passes) 1192 against 754 us.
+// own expert's, are beside it.  (The passes of a tile over the same weights walk them together.)  Measured at E = 8,
+// H = 4096, F = 14336, one row an expert: 591 us for both products in step, 487 us started apart (5.8 TB/s of weights);
+// 718 / 558 us with non-temporal loads (each 128-byte line is asked for in two halves, which a cached load fetches once).
+//
+// Against the 256-row tiles (split last rounds included), bf16, both products, us, tiles -> here; "routed" is the top-K
+// of random logits, "skewed" the same with a Zipf(1.1) bias on the experts:
+//   rows an expert, mean    1 each       16 routed   16 skewed   24 routed   24 skewed   28 routed   32 each    64 each
+//   E 8,   H 4096, F 14336  643 -> 485   630 -> 563  635 -> 595  637 -> 602  641 -> 696  638 -> 654  636 -> 634  651 -> 806
+//   E 128, H 2048, F 768    303 -> 210   308 -> 263  211 -> 212  308 -> 288  244 -> 256  310 -> 307  313 -> 297  343 -> 393
+//   E 32,  H 2048, F 4096   404 -> 269   404 -> 323  384 -> 353  402 -> 360  375 -> 375  404 -> 383  409 -> 368  409 -> 461
+// With passes of 32 rows an expert's further rows cost as many more streams of its weights: 24 skewed 777, 288 and 426.
+// Routings that put nearly all rows on a few of many experts are what is left to the tiles' favour (E 128, Zipf(2), 16
+// rows: 118 -> 148).  fp32, E = 8, H = 1024, F = 4096, one row each, against its 128-row tiles: 463 -> 77 us; its sums
+// are slow enough that rows and not weights bound a pass, and it keeps 32 of them.
 #include <algorithm>
 
 #include "common.h"
@@ -218,9 +226,16 @@ __device__ __forceinline__ void small_pass(const SmallArgs& g, const uint8_t* ba
   }
 }
 
+// Rows of a pass: 64 take 250 registers of the 256 that two waves a SIMD have (NF = 4).
+template <bool F32>
+constexpr int pass_rows() {
+  return F32 ? 32 : 64;
+}
+
 template <bool F32, bool GU, int NF, int NW>
 __global__ __launch_bounds__(NW * 64, 8 / NW) void k_gemm_small(SmallArgs g) {
   __shared__ __attribute__((aligned(16))) float red[NW * 16 * (NF * 16 + 4)];
+  constexpr int PR = pass_rows<F32>();
   const int slot = (int)(blockIdx.x / g.Tn), nt = (int)(blockIdx.x % g.Tn);
   int e = slot, pass = 0;
   if (slot >= g.E) {  // the (slot - E)-th of the passes past the experts' first ones
@@ -229,7 +244,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void k_gemm_small(SmallArgs g) {
     for (int e0 = 0;; e0 += 64) {
       if (e0 >= g.E) return;
       const int i = e0 + lane;
-      const int c = i < g.E ? max((g.offsets[i + 1] - g.offsets[i] + 31) / 32 - 1, 0) : 0;
+      const int c = i < g.E ? max((g.offsets[i + 1] - g.offsets[i] + PR - 1) / PR - 1, 0) : 0;
       int upto = c;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
@@ -248,13 +263,14 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void k_gemm_small(SmallArgs g) {
     e = __builtin_amdgcn_readfirstlane(e);
     pass = __builtin_amdgcn_readfirstlane(pass);
   }
-  const int m0 = g.offsets[e] + pass * 32, hi = g.offsets[e + 1];
+  const int m0 = g.offsets[e] + pass * PR, hi = g.offsets[e + 1];
   if (m0 >= hi) return;
   const int n0 = nt * NF * (GU ? 8 : 16);
   const uint8_t* const b0 = g.B + (int64_t)e * g.b_ebytes;
   const uint8_t* const b1 = GU ? g.B2 + (int64_t)e * g.b_ebytes : nullptr;
   const uint32_t tile = (uint32_t)(e * g.Tn + nt);
-  if (hi - m0 > 16) small_pass<F32, GU, NF, NW, 2>(g, b0, b1, m0, min(32, hi - m0), n0, tile, red);
+  if (PR > 32 && hi - m0 > 32) small_pass<F32, GU, NF, NW, PR / 16>(g, b0, b1, m0, min(PR, hi - m0), n0, tile, red);
+  else if (hi - m0 > 16) small_pass<F32, GU, NF, NW, 2>(g, b0, b1, m0, min(32, hi - m0), n0, tile, red);
   else small_pass<F32, GU, NF, NW, 1>(g, b0, b1, m0, hi - m0, n0, tile, red);
 }
 
@@ -263,7 +279,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void k_gemm_small(SmallArgs g) {
 template <bool F32, bool GU>
 int launch_small(const char* name, hipStream_t s, SmallArgs a, int64_t E, int64_t R) {
   a.E = (int)E;
-  const int64_t slots = E + R / 32;  // every expert's first pass, and as many more as R rows can need
+  const int64_t slots = E + R / pass_rows<F32>();  // every expert's first pass, and as many more as R rows can need
   if (cdiv(a.N, GU ? 32 : 64) * E >= 512) {
     a.Tn = cdiv(a.N, GU ? 32 : 64);
     MOE_LAUNCH(name, (k_gemm_small<F32, GU, 4, 4>), dim3((unsigned)(a.Tn * slots)), dim3(256), 0, s, a);
@@ -275,11 +291,12 @@ int launch_small(const char* name, hipStream_t s, SmallArgs a, int64_t E, int64_
 }
 }  // namespace
 
-// Up to 24 rows an expert on average (fp32: 32): few passes past the first, (1 + R / 32E) of the weights' stream at the
-// most (figures at the top).  A weight slice is addressed by 32-bit byte offsets.
+// Up to 24 rows an expert on average (fp32: 32): routed rows gain 6-16% there on every layer measured and nothing at 28;
+// skewed ones gain up to 16 and give back at most 9% at 24 (figures at the top).  The host does not know the rows of each
+// expert.  A weight slice and a pass's rows are addressed by 32-bit byte offsets.
 bool swiglu_small_takes(int64_t R, int64_t H, int64_t F, int64_t E, int elem) {
   const int64_t lim = (int64_t)1 << 32;
-  return R <= (elem == 4 ? 32 : 24) * E && H * F * elem < lim && 32 * std::max(H, F) * elem < lim &&
+  return R <= (elem == 4 ? 32 : 24) * E && H * F * elem < lim && 64 * std::max(H, F) * elem < lim &&
          (E + R / 32) * std::max((F + 15) / 16, (H + 31) / 32) < ((int64_t)1 << 31);
 }
 

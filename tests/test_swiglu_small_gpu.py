@@ -1,4 +1,4 @@
-"""The forward products for few rows per expert (csrc/gemm_small.hip): segments at the edges of the 16- and 32-row
+"""The forward products for few rows per expert (csrc/gemm_small.hip): segments at the edges of the 16-, 32- and 64-row
 passes, rows of one partial 128-byte chunk and of many, both column widths of a block, against float64."""
 
 from __future__ import annotations
@@ -24,6 +24,8 @@ CASES = [
     ("bf16", 64, 64, [0] * 70 + [300] + [0, 33] * 40),  # most rows on one expert past the first 64
     ("f32", 1004, 160, [0, 65, 100, 1, 16, 9]),
     ("f32", 132, 4128, [1, 17, 32, 48]),
+    ("bf16", 200, 96, [34, 48, 49, 63, 65, 128, 129, 1] + [0] * 20),  # 64-row passes: partial, whole, several
+    ("bf16", 1032, 4128, [50, 0, 0, 0, 66, 0, 0]),  # ... over many columns: 64 weight rows a block
 ]
 
 
