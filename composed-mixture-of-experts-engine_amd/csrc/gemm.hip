@@ -1263,18 +1263,20 @@ int launch(const char* name, hipStream_t s, const GemmArgs& a, int64_t R) {
   return check_launch(name);
 }
 
-// Room for the partial tiles of an XCD, for a product of R rows and N columns: 8 a tile, at most kSplitMax.
+// Room for the partial tiles of an XCD, for a product of R rows and N columns: 8 a tile, at most kSplitMax.  None for a
+// product of 16 rounds of tiles or more, of which the last is too little to pay for the extra launches.
 int split_parts(int64_t R, int64_t E, int64_t N) {
   const int64_t tiles = ((R + GBM - 1) / GBM + E) * ((N + GBN - 1) / GBN);
   return (int)std::min<int64_t>(kSplitMax, 8 * ((tiles + 7) / 8));
 }
 size_t split_bytes(int64_t R, int64_t E, int64_t N) {
+  if (R <= 0 || E <= 0 || R / GBM * ((N + GBN - 1) / GBN) >= 16 * 256) return 0;
   return (size_t)8 * split_parts(R, E, N) * GBM * GBN * sizeof(float);
 }
 // The caller's workspace past its first `used` bytes, for the partial tiles; too small: the product is not split.
-// Neither is one of 16 rounds of tiles or more, of which the last is too little to pay for the extra launches.
 void take_split(GemmArgs& a, int64_t R, void* ws, size_t ws_bytes, size_t used) {
-  if (R / GBM * ((a.N + GBN - 1) / GBN) >= 16 * 256 || ws_bytes < used + split_bytes(R, a.E, a.N)) return;
+  const size_t need = split_bytes(R, a.E, a.N);
+  if (need == 0 || ws_bytes < used + need) return;
   a.part = reinterpret_cast<float*>(static_cast<char*>(ws) + used);
   a.npart = split_parts(R, a.E, a.N);
 }
@@ -1291,7 +1293,20 @@ using namespace moe;
 extern "C" size_t moe_swiglu_workspace(int64_t E) { return (size_t)((2 * E + 1) * 4 + 255) & ~(size_t)255; }
 
 extern "C" size_t moe_swiglu_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E) {
-  return R > 0 && E > 0 && !swiglu_small_takes(R, H, F, E, 2) ? split_bytes(R, E, H) : 0;
+  (void)F;
+  return split_bytes(R, E, H);  // dxp is H wide, as the down projection is
+}
+
+// With few rows an expert the e4m3 down projection is bound by its weights' stream and the two more launches cost what
+// the split gains: E = 8, H = 4096, F = 14336 392 -> 393 us a forward at 4 to 24 rows, E = 128, H = 2048, F = 768 (whole
+// rounds, nothing to split) 200 -> 206, E = 8, H = 1024, F = 4096 75 -> 70.  dxp, with twice the slices, gains there:
+// backward 1500 -> 1265, 613 -> 616, 263 -> 161.
+extern "C" size_t moe_swiglu_fwd_fp8_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E) {
+  return R <= 24 * E ? 0 : moe_swiglu_split_workspace(R, H, F, E);
+}
+
+extern "C" size_t moe_swiglu_fwd_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E) {
+  return swiglu_small_takes(R, H, F, E, 2) ? 0 : split_bytes(R, E, H);
 }
 
 extern "C" int moe_swiglu_fwd(const void* xp, const void* w_gate, const void* w_up, const void* w_down,

@@ -458,17 +458,18 @@ int launch_f32(const char* name, hipStream_t s, const GemmF32Args& a, int64_t R)
 }
 
 // Partial tiles: 16 a tile, at most kSplitMaxF32 an XCD; none for a product of 16 rounds or more, or where the caller's
-// workspace ends at the tables.  cols: columns of the product's tiles (2F for the gate/up product).
+// workspace has no room for them.  cols: columns of the product's tiles (2F for the gate/up product).
 int split_parts_f32(int64_t R, int64_t E, int64_t cols) {
   const int64_t tiles = ((R + FBM - 1) / FBM + E) * ((cols + FBN - 1) / FBN);
   return (int)std::min<int64_t>(kSplitMaxF32, 16 * ((tiles + 7) / 8));
 }
 size_t split_bytes_f32(int64_t R, int64_t E, int64_t cols) {
+  if (R <= 0 || E <= 0 || R / FBM * ((cols + FBN - 1) / FBN) >= 16 * 512) return 0;
   return (size_t)8 * split_parts_f32(R, E, cols) * FBM * FBN * sizeof(float);
 }
 void take_split_f32(GemmF32Args& a, int64_t R, int64_t cols, void* ws, size_t ws_bytes) {
-  const size_t used = moe_swiglu_f32_workspace(a.E);
-  if (R / FBM * ((cols + FBN - 1) / FBN) >= 16 * 512 || ws_bytes < used + split_bytes_f32(R, a.E, cols)) return;
+  const size_t used = moe_swiglu_f32_workspace(a.E), need = split_bytes_f32(R, a.E, cols);
+  if (need == 0 || ws_bytes < used + need) return;
   a.part = reinterpret_cast<float*>(static_cast<char*>(ws) + used);
   a.npart = split_parts_f32(R, a.E, cols);
 }
@@ -487,7 +488,13 @@ using namespace moe;
 extern "C" size_t moe_swiglu_f32_workspace(int64_t E) { return (size_t)((E + 1) * 4 + 255) & ~(size_t)255; }
 
 extern "C" size_t moe_swiglu_f32_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E) {
-  return R > 0 && E > 0 ? split_bytes_f32(R, E, std::max(H, 2 * F)) : 0;
+  // the most that one of the products takes: 2F (gate/up), F (dact) or H columns (the others), each by its own size
+  return std::max({split_bytes_f32(R, E, 2 * F), split_bytes_f32(R, E, F), split_bytes_f32(R, E, H)});
+}
+
+extern "C" size_t moe_swiglu_fwd_f32_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E) {
+  if (swiglu_small_takes(R, H, F, E, 4)) return 0;
+  return std::max(split_bytes_f32(R, E, 2 * F), split_bytes_f32(R, E, H));
 }
 
 extern "C" int moe_swiglu_fwd_f32(const float* xp, const float* w_gate, const float* w_up, const float* w_down,

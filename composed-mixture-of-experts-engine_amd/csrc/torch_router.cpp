@@ -393,9 +393,12 @@ at::Tensor op_unpermute_sum(const at::Tensor& dxp_in, const OptTensor& addend_in
 }
 
 // Bytes of the grouped GEMM's tile tables and of the partial tiles of products split over k.
-size_t gemm_workspace(bool f32, int64_t R, int64_t H, int64_t F, int64_t E) {
-  return f32 ? moe_swiglu_f32_workspace(E) + moe_swiglu_f32_split_workspace(R, H, F, E)
-             : moe_swiglu_workspace(E) + moe_swiglu_split_workspace(R, H, F, E);
+size_t gemm_workspace(bool f32, bool fwd, int64_t R, int64_t H, int64_t F, int64_t E) {
+  if (f32)
+    return moe_swiglu_f32_workspace(E) +
+           (fwd ? moe_swiglu_fwd_f32_split_workspace(R, H, F, E) : moe_swiglu_f32_split_workspace(R, H, F, E));
+  return moe_swiglu_workspace(E) +
+         (fwd ? moe_swiglu_fwd_split_workspace(R, H, F, E) : moe_swiglu_split_workspace(R, H, F, E));
 }
 
 std::tuple<at::Tensor, OptTensor, at::Tensor> op_swiglu_forward(const at::Tensor& xp, const at::Tensor& wg,
@@ -407,7 +410,7 @@ std::tuple<at::Tensor, OptTensor, at::Tensor> op_swiglu_forward(const at::Tensor
   at::Tensor act = at::empty({R, F}, xp.options()), y = at::empty({R, H}, xp.options());
   OptTensor hgu;
   if (keep_preact) hgu = at::empty({R, 2 * F}, xp.options());
-  const size_t nbytes = gemm_workspace(f32, R, H, F, E);
+  const size_t nbytes = gemm_workspace(f32, true, R, H, F, E);
   const at::Tensor ws = scratch(nbytes, xp);
   const hipStream_t s = stream_of(xp);
   void* const h = const_cast<void*>(ptr(hgu));
@@ -431,7 +434,7 @@ std::vector<at::Tensor> op_swiglu_backward(const at::Tensor& dy, const at::Tenso
   const int64_t R = xp.size(0), H = xp.size(1), E = wg.size(0), F = wg.size(1);
   at::Tensor dh = at::empty({R, 2 * F}, xp.options()), dxp = at::empty({R, H}, xp.options());
   at::Tensor dwg = at::empty_like(wg), dwu = at::empty_like(wu), dwd = at::empty_like(wd);
-  const size_t nbytes = gemm_workspace(f32, R, H, F, E);
+  const size_t nbytes = gemm_workspace(f32, false, R, H, F, E);
   const at::Tensor ws = scratch(nbytes, xp);
   const hipStream_t s = stream_of(xp);
   if (f32)

@@ -433,7 +433,7 @@ def swiglu_forward_fp8(xq, sx, wq, wscale, offsets, out_dtype=torch.bfloat16, ke
     hgu = torch.empty((R, 2 * F), dtype=out_dtype, device=dev) if keep_preact else None
     y = torch.empty((R, H), dtype=out_dtype, device=dev)
     lib = L.load()
-    nbytes = lib.moe_swiglu_fwd_fp8_workspace(R, F, E) + lib.moe_swiglu_split_workspace(R, H, F, E)
+    nbytes = lib.moe_swiglu_fwd_fp8_workspace(R, F, E) + lib.moe_swiglu_fwd_fp8_split_workspace(R, H, F, E)
     ws = L.workspace(nbytes, dev)
     rc = lib.moe_swiglu_fwd_fp8(
         xq.data_ptr(), sx.contiguous().data_ptr(), wg.data_ptr(), sg.contiguous().data_ptr(), wu.data_ptr(),

@@ -255,10 +255,14 @@ int moe_unpermute_sum(const void* dxp, const void* addend, int dtype, const int3
  * Limits: H % 8 == 0, F % 32 == 0, E <= 1024.
  * ---------------------------------------------------------------------- */
 size_t moe_swiglu_workspace(int64_t E);
-/* Bytes that moe_swiglu_fwd, moe_swiglu_bwd and moe_swiglu_fwd_fp8 use beyond their own workspace size, if the
- * caller passes that much more (ws_bytes): partial tiles of products whose last round of tiles is split over k.
- * Without them the same products run unsplit. */
+/* Bytes that moe_swiglu_bwd and moe_swiglu_fwd_fp8 use beyond their own workspace size, if the caller passes that
+ * much more (ws_bytes): partial tiles of products whose last round of tiles is split over k.  Without them the same
+ * products run unsplit; 0: they are not split.  moe_swiglu_fwd_split_workspace and
+ * moe_swiglu_fwd_fp8_split_workspace: what to pass moe_swiglu_fwd, which uses none for few rows per expert, and
+ * moe_swiglu_fwd_fp8, to which it is of no use there. */
 size_t moe_swiglu_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E);
+size_t moe_swiglu_fwd_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E);
+size_t moe_swiglu_fwd_fp8_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E);
 int moe_swiglu_fwd(const void* xp, const void* w_gate, const void* w_up, const void* w_down,
                    const int32_t* offsets, int64_t R, int64_t H, int64_t F, int64_t E,
                    void* act, void* hgu, void* y, void* workspace, size_t ws_bytes, void* stream);
@@ -272,7 +276,9 @@ int moe_swiglu_bwd(const void* dy, const void* xp, const void* act, const void* 
  * moe_layer.py L:166-198, L:326-337).  Limits: H % 4 == 0, F % 32 == 0, E <= 1024; the operands 16-byte
  * aligned.  Workspace: moe_swiglu_f32_workspace(E) bytes. */
 size_t moe_swiglu_f32_workspace(int64_t E);
-size_t moe_swiglu_f32_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E); /* as moe_swiglu_split_workspace */
+/* As moe_swiglu_split_workspace (enough for either direction) and moe_swiglu_fwd_split_workspace. */
+size_t moe_swiglu_f32_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E);
+size_t moe_swiglu_fwd_f32_split_workspace(int64_t R, int64_t H, int64_t F, int64_t E);
 int moe_swiglu_fwd_f32(const float* xp, const float* w_gate, const float* w_up, const float* w_down,
                        const int32_t* offsets, int64_t R, int64_t H, int64_t F, int64_t E,
                        float* act, float* hgu, float* y, void* workspace, size_t ws_bytes, void* stream);

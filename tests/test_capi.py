@@ -103,3 +103,23 @@ def test_torch_binding_loads_and_shares_the_library():
     assert os.path.realpath(_lib.LIB_PATH) in maps
     with pytest.raises(RuntimeError, match="AMD Instinct GPU"):
         R.RouterCore.apply(torch.zeros(4, 8), torch.zeros(8, 2), 1, 0.0, 0.0, None)
+
+
+def test_split_workspace_is_each_products_own():
+    """Room for partial tiles is asked for where a call uses it: none for a bf16 or fp32 forward that takes the few-row
+    kernel, nor an e4m3 forward that does not gain by it, none for products of 16 rounds of tiles or more, and else what they use."""
+    lib = _lib.load()
+    tile = 256 * 256 * 4
+    for R, E in ((32, 8), (1, 8), (24 * 128, 128)):  # few rows an expert
+        assert lib.moe_swiglu_fwd_split_workspace(R, 4096, 14336, E) == 0
+        assert lib.moe_swiglu_fwd_f32_split_workspace(R, 1024, 4096, E) == 0
+        assert lib.moe_swiglu_fwd_fp8_split_workspace(R, 4096, 14336, E) == 0
+        assert lib.moe_swiglu_split_workspace(R, 4096, 14336, E) >= 8 * 8 * tile
+        assert lib.moe_swiglu_f32_split_workspace(R, 1024, 4096, E) > 0
+    assert lib.moe_swiglu_split_workspace(262144, 2048, 768, 128) == 0  # 32 rounds
+    assert lib.moe_swiglu_fwd_split_workspace(262144, 2048, 768, 128) == 0
+    assert lib.moe_swiglu_f32_split_workspace(1 << 20, 1024, 1024, 8) == 0
+    ordinary = lib.moe_swiglu_split_workspace(16384, 4096, 14336, 8)
+    assert ordinary > 0 and lib.moe_swiglu_fwd_fp8_split_workspace(16384, 4096, 14336, 8) == ordinary
+    assert lib.moe_swiglu_fwd_split_workspace(16384, 4096, 14336, 8) == ordinary
+    assert lib.moe_swiglu_split_workspace(0, 4096, 14336, 8) == 0

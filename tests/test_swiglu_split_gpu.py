@@ -22,6 +22,8 @@ CASES = [
     (512, 96, [700]),
     (1032, 3104, [257, 513, 40, 0]),
     (4096, 1056, [600] * 30),
+    (1024, 2080, [20, 3, 0, 33]),  # few rows: dxp is split (the forward takes the few-row kernel)
+    (4096, 4096, [4, 4]),
 ]
 
 
@@ -77,7 +79,16 @@ def test_split_products(case):
 
 def test_split_fp8():
     """The e4m3 down projection, split and whole: the same sums in another order, so within one bf16 rounding."""
-    H, Fd, counts = 1024, 4096, [300, 17, 0, 511]
+    _fp8(1024, 4096, [300, 17, 0, 511])
+
+
+@pytest.mark.parametrize("H,Fd,counts", [(4096, 8192, [4, 4]), (1040, 4128, [20, 3, 0, 33])])
+def test_split_fp8_few_rows(H, Fd, counts):
+    """The same with few rows, where the operation leaves it whole but a caller of the C ABI may pass the room."""
+    _fp8(H, Fd, counts, room=True)
+
+
+def _fp8(H, Fd, counts, room=False):
     E, R = len(counts), sum(counts)
     g = torch.Generator(device=dev()).manual_seed(7)
     ws = [torch.randn(E, Fd, H, generator=g, device=dev()) * H**-0.5, torch.randn(E, Fd, H, generator=g, device=dev())
@@ -89,10 +100,12 @@ def test_split_fp8():
     lib = L.load()
     assert lib.moe_swiglu_split_workspace(R, H, Fd, E) > 0
     n = lib.moe_swiglu_fwd_fp8_workspace(R, Fd, E)
-    wsp = torch.empty(n, dtype=torch.uint8, device=dev())
+    more = lib.moe_swiglu_split_workspace(R, H, Fd, E)
+    wsp = torch.empty(n + more, dtype=torch.uint8, device=dev())
     y0 = torch.empty_like(y)
-    _call(lib.moe_swiglu_fwd_fp8, xq.data_ptr(), sx.data_ptr(), *[t.data_ptr() for pair in q for t in pair],
-          offs.data_ptr(), R, H, Fd, E, None, None, y0.data_ptr(), wsp.data_ptr(), n, L.stream_of(dev()))
+    for out, nbytes in ([(y, n + more)] if room else []) + [(y0, n)]:
+        _call(lib.moe_swiglu_fwd_fp8, xq.data_ptr(), sx.data_ptr(), *[t.data_ptr() for pair in q for t in pair],
+              offs.data_ptr(), R, H, Fd, E, None, None, out.data_ptr(), wsp.data_ptr(), nbytes, L.stream_of(dev()))
     torch.cuda.synchronize()
     a, b = y.double(), y0.double()
     # fp32 sums of 4096 terms differ by at most 2 x 4096 x 2^-24 of the sum of magnitudes, here below 8 rms of y
