@@ -111,10 +111,12 @@ ROUTE_SHAPES = [
     (1000, 2048, 16, 4, torch.bfloat16),   # E = 16
     (129, 512, 5, 2, torch.bfloat16),      # E < 8, ragged block
     (40, 256, 12, 12, torch.bfloat16),     # K == E
-    (200, 520, 8, 2, torch.bfloat16),      # H % 256 != 0: fused forward, backward through the router kernels
+    (200, 520, 8, 2, torch.bfloat16),      # H % 256 != 0: a partial slice in both fused kernels
     (300, 2048, 64, 6, torch.bfloat16),    # E = 64: wide router kernel over xn
     (200, 512, 8, 2, torch.float32),       # fp32: generic router over xn
 ]
+# bf16 with few experts whose gate image does not fit in LDS (H > 4096): the norm kernels and the router kernels
+WIDE_SHAPES = [(100, 4104, 8, 2, torch.bfloat16), (70, 8192, 16, 4, torch.bfloat16)]
 
 
 def _rid(s):
@@ -127,7 +129,7 @@ def _gate(H, E, dtype, seed):
     return (torch.randn(H, E, generator=g) * 0.02 * math.sqrt(4096.0 / H)).to(dtype)
 
 
-@pytest.mark.parametrize("shape", ROUTE_SHAPES, ids=_rid)
+@pytest.mark.parametrize("shape", ROUTE_SHAPES + WIDE_SHAPES, ids=_rid)
 def test_norm_router_forward_parity(shape):
     N, H, E, K, xd = shape
     say(f"[norm router fwd] {_rid(shape)}")
@@ -165,7 +167,7 @@ def test_norm_router_forward_parity(shape):
 
 
 @pytest.mark.parametrize("expert_grad", [True, False], ids=["with_dxn", "router_only"])
-@pytest.mark.parametrize("shape", ROUTE_SHAPES[:6], ids=_rid)
+@pytest.mark.parametrize("shape", ROUTE_SHAPES[:6] + WIDE_SHAPES, ids=_rid)
 def test_norm_router_backward_parity(shape, expert_grad):
     """NormRouterCore's gradients against the chain rule over the oracle: the router backward on xn (oracle
     router_full with the kernel's routing), its dxn plus an expert-path gradient of xn (or none), then the

@@ -6,12 +6,34 @@ from __future__ import annotations
 import pytest
 import torch
 
-from gpu_util import dev, say
+from gpu_util import TOL, assert_rel, dev, say
 
 from moe_mi355 import _lib as L
 from moe_mi355 import ops
 
 pytestmark = pytest.mark.gpu
+
+
+
+def _splits(counts, N, nk):
+    """(whole tiles, tiles split, S) of each XCD of a row-grouped product N columns wide with nk k slices: the host's copy
+    of the kernels' rule (split_parts, split_of and the tile ranges in csrc/gemm.hip)."""
+    R, E, cols = sum(counts), len(counts), -(-N // 256)
+    npart = min(64, 8 * -(-((-(-R // 256) + E) * cols) // 8))
+    total = sum(-(-c // 256) for c in counts) * cols
+    chunk, out = -(-total // 8), []
+    for xcd in range(8):
+        n = max(0, min(chunk, total - xcd * chunk))
+        r, best, cost = n & 31, 1, nk
+        for S in range(2, 9):
+            if r * S > npart or S > nk:
+                break
+            c = ((r * S + 31) >> 5) * (-(-nk // S) + 20) + 5
+            if c < cost:
+                best, cost = S, c
+        out.append((n - r, r, best if r else 1))
+    return out
+
 
 # (H, F, rows of each expert): one or several m-tiles an expert, ragged ones, k past and short of whole 64-wide slices,
 # dxp's change of weights inside a slice (F % 64 == 32) and inside a part, a width that is no multiple of the tile,
@@ -24,14 +46,33 @@ CASES = [
     (4096, 1056, [600] * 30),
     (1024, 2080, [20, 3, 0, 33]),  # few rows: dxp is split (the forward takes the few-row kernel)
     (4096, 4096, [4, 4]),
+    # whole rounds and a few tiles more, which are split (33 to 36 tiles an XCD)
+    (4096, 4096, [256 * 15, 300]),
+    (4088, 4128, [256 * 14 + 100, 511]),
+    (2048, 4160, [255] * 31 + [0, 500]),
 ]
+ROUND_AND_PARTS = CASES[-3:]
+# which of the down projection (y) and dxp (d) the rule splits in a case; the others run whole with the room for it as
+# without, and with few rows the forward takes the few-row kernel instead
+SPLIT = {(512, 96): "", (4096, 1056): "", (4096, 4096): "yd", (1024, 2080): "yd", (256, 4096): "yd", (264, 2080): "yd",
+         (1032, 3104): "yd", (4088, 4128): "yd", (2048, 4160): "yd"}
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"H{c[0]}-F{c[1]}-E{len(c[2])}-R{sum(c[2])}")
+def test_cases_split_what_they_say(case):
+    H, Fd, counts = case
+    y, d = _splits(counts, H, -(-Fd // 64)), _splits(counts, H, -(-2 * Fd // 64))
+    for name, ranges in (("y", y), ("d", d)):
+        assert any(S > 1 for _, _, S in ranges) == (name in SPLIT[(H, Fd)])
+    if case in ROUND_AND_PARTS:
+        assert any(S > 1 and full > 0 for full, _, S in y) and any(S > 1 and full > 0 for full, _, S in d)
 
 
 def _call(fn, *args):
     L.check(fn(*args), "call")
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: f"H{c[0]}-F{c[1]}-E{len(c[2])}")
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"H{c[0]}-F{c[1]}-E{len(c[2])}-R{sum(c[2])}")
 def test_split_products(case):
     H, Fd, counts = case
     E, R = len(counts), sum(counts)
@@ -80,6 +121,12 @@ def test_split_products(case):
 def test_split_fp8():
     """The e4m3 down projection, split and whole: the same sums in another order, so within one bf16 rounding."""
     _fp8(1024, 4096, [300, 17, 0, 511])
+
+
+def test_split_fp8_after_whole_rounds():
+    H, Fd, counts = 4096, 8192, [256 * 15, 300]
+    assert any(S > 1 and full > 0 for full, _, S in _splits(counts, H, Fd // 128))
+    _fp8(H, Fd, counts)
 
 
 @pytest.mark.parametrize("H,Fd,counts", [(4096, 8192, [4, 4]), (1040, 4128, [20, 3, 0, 33])])
@@ -164,4 +211,12 @@ def test_split_products_f32(case):
                 bound = bound + (H + 16) * 2.0**-24 * 4 * mag
             for t in (got, other):
                 assert bool(((t[lo:hi].double() - want).abs() <= bound).all())
-        assert bool(torch.isfinite(dwg[e]).all()) and bool(torch.allclose(dwd[e], dws[2][e], rtol=0, atol=1e-4))
+        # the weights' gradients, from dh and act of the split products and of the whole ones
+        gate, up = x @ wg[e].double().t(), x @ wu[e].double().t()
+        sg = torch.sigmoid(gate)
+        da = dy[lo:hi].double() @ d
+        for got, whole, want in ((dwg[e], dws[0][e], (da * up * sg * (1 + gate * (1 - sg))).t() @ x),
+                                 (dwu[e], dws[1][e], (da * gate * sg).t() @ x),
+                                 (dwd[e], dws[2][e], dy[lo:hi].double().t() @ (gate * sg * up))):
+            assert_rel(got, want, TOL[torch.float32], "dW")
+            assert_rel(whole, want, TOL[torch.float32], "dW of whole tiles")
