@@ -179,8 +179,8 @@ __global__ __launch_bounds__(FNT, 2) void k_gemm_f32(GemmF32Args g) {
   const int nlen = (EPI == 1) ? min(FBN, 2 * (g.F - nt * (FBN / 2))) : min(FBN, g.N - n0);
   const int nk = (klen + FBK - 1) / FBK;
 
-  // ---- operand sources.  Rows mode: thread q = tid + 256 j loads row q / 4, k chunk (q % 4) * 4 of the slice;
-  // cols mode: k-row q / 32, i chunk (q % 32) * 4.  Rows / columns past the tile are clamped to valid ones
+  // ---- operand sources, FNJ 16-byte units q = tid + FNT j a thread.  Rows mode: row q / FCH, k chunk (q % FCH) * 4 of
+  // the slice; cols mode: k-row q / 32, i chunk (q % 32) * 4.  Rows / columns past the tile are clamped to valid ones
   // (their results are never stored); k past the reduction reads zeros. ----
   const float* arow[FNJ];
   const float* brow[FNJ];
@@ -236,8 +236,8 @@ __global__ __launch_bounds__(FNT, 2) void k_gemm_f32(GemmF32Args g) {
         const int k = k0 + (q >> 5);
         const float* src;
         if constexpr (GROUP == 0) {
-          // both j of a thread share its column (256 is a multiple of 32), so the second source's column base
-          // b2row0 serves both
+          // all units of a thread share its column (FNT is a multiple of 32), so the second source's column base
+          // b2row0 serves them all
           if (g.b_split > 0 && k >= bsplit) src = b2row0 + (int64_t)(k - bsplit) * g.ldb;
           else src = brow[j] + (int64_t)k * g.ldb;
         } else {

@@ -271,9 +271,6 @@ class Plan:
     def rows(self) -> int:
         return self.N * self.K
 
-    def drop_u8(self):
-        return None if self.drop is None else self.drop.view(torch.uint8)
-
 
 def cumcount(groups: torch.Tensor) -> torch.Tensor:
     """Each element's 0-based position among the earlier elements of its group, for any int64 group ids
