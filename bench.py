@@ -337,6 +337,7 @@ def run_c1(args, torch, with_cpu=True):
 # ---------------------------------------------------------------------------
 GEMM_KERNELS = ("k_gemm_swiglu_fwd1", "k_gemm_swiglu_fwd2", "k_gemm_swiglu_dact", "k_gemm_swiglu_dxp",
                 "k_gemm_swiglu_dwd", "k_gemm_swiglu_dw1")
+GEMM_SPLIT_KERNELS = ("k_gemm_parts", "k_gemm_reduce", "k_gemm_reduce_f32")
 
 
 def gemm_flops(R, H, F):
@@ -426,7 +427,9 @@ def run_layer(args, torch, cfg, layout, inp, default_numerics=False):
     dom = max((k for k in kernels if k in fl), key=lambda k: kernels[k]["avg_us"] * kernels[k]["launches"])
     achieved = kernels[dom]["TFLOPs"]
     step_flops = 18 * R * cfg.H * cfg.F
+    # one launch of each product a step, and the launches of products whose last round of tiles is split
     gemm_ms = sum(prof[k][1] / prof[k][0] for k in fl if k in prof)
+    gemm_ms += sum(prof[k][1] for k in GEMM_SPLIT_KERNELS if k in prof) / prof[dom][0]
     res = {
         "workload": f"{cfg.name} layer fwd+bwd ({layout} layout)", "tokens": cfg.T, "d_model": cfg.H,
         "experts": cfg.E, "ffn": cfg.F, "top_k": cfg.K, "rows_computed": R,
